@@ -115,3 +115,25 @@ def test_midb_refuses_what_it_does_not_take():
     gx, gxs, gw, gws = to_gpu(x, xs, w, ws)
     with pytest.raises(ValueError):
         wave_amd.mxfp4_gemm(gx, gxs, gw, gws, out, variant=V, split_k=1)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(1, 160, 2048), (96, 2048, 2048), (128, 8192, 4096), (129, 160, 1024), (256, 12288, 3072)])
+def test_midb_shuffled_scales_in_place(m, n, k, dt):
+    """Scales in e8m0_shuffle order read in place (no scratch): the bits of the call with MFMA32 scales, at both block
+    heights, a row count that leaves the last 32-row block almost empty, N ending inside a strip, one and several turns
+    of the ring; also what the library's own choice runs from N = 8192 / 12288 on."""
+    x, xs, w, ws = orc.make_inputs(m, n, k, seed=m + n, scale_lo=100, scale_hi=154)
+    gx, gxs, gw, gws = to_gpu(x, xs, w, ws)
+    gwp = wave_amd.b_preshuffle(gw)
+    got = []
+    for layout in (_lib.SCALE_E8M0_SHUFFLE, _lib.SCALE_MFMA32):
+        sa = wave_amd.scale_convert(gxs, m, k // 32, _lib.SCALE_ROW_MAJOR, layout)
+        sb = wave_amd.scale_convert(gws, n, k // 32, _lib.SCALE_ROW_MAJOR, layout)
+        for kw in (dict(variant=V, workspace=False, split_k=1), dict()):
+            if kw or n >= 8192:
+                out = torch.full((m, n), float("nan"), dtype=dt, device=DEV)
+                wave_amd.mxfp4_gemm(gx, sa, gwp, sb, out, b_layout=_lib.B_PRESHUFFLE, a_scale_layout=layout, b_scale_layout=layout, **kw)
+                got.append(out.float().cpu().numpy())
+    assert all(np.array_equal(g, got[0]) for g in got)
+    assert_close(got[0], c_oracle.scaled_gemm_exact(x, w, xs, ws), dt, f"{m}x{n}x{k}")

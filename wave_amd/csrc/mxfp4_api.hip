@@ -606,14 +606,18 @@ int wave_mxfp4_gemm(const void *a, const void *a_scale, const void *b, const voi
   const int64_t cus_n = 128 * (int64_t)device_cus();  // columns of one round of strips
   // (with resident scales and K <= 4096 it leads from N = 8192 on for 48 rows and more: 128 x 8192 x 4096 15.5 -> 12.5,
   // 48 rows 12.4 -> 11.2, 256 rows 20.0 -> 18.0; at N = 4096 the 128x128 tiles are level or ahead)
-  const int64_t midb_min_n = native_scales && k <= 4096 && m >= 48 ? 8192 : 12288;
+  // Both tensors in e8m0_shuffle order, the reference's preshuffled format, are read in place at the same speed (us,
+  // this kernel / the strip kernel on the same operands: 128 x 28672 x 8192 27.2 / 30.6, 64 x 14336 x 4096 12.2 / 13.1,
+  // 128 x 8192 x 4096 12.8 / 15.5; the re-layout launch in front of it cost 256 x 28672 x 8192 50.1 instead of 40.7).
+  const bool both_shuffled = a_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE && b_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE;
+  const bool midb_in_place = native_scales || both_shuffled;
+  const int64_t midb_min_n = midb_in_place && k <= 4096 && m >= 48 ? 8192 : 12288;
   if (variant == WAVE_MXFP4_VARIANT_AUTO && n >= midb_min_n && split_k <= 1 && midb_shape_ok(m, n, k, b_layout) &&
       (m > 128 ? n <= cus_n
-               : native_scales && n <= 2 * cus_n && (m >= 64 || (m >= 32 && n <= cus_n && (n >= 20480 || k <= 4096)))))
+               : midb_in_place && n <= 2 * cus_n && (m >= 64 || (m >= 32 && n <= cus_n && (n >= 20480 || k <= 4096)))))
     v = WAVE_MXFP4_VARIANT_MID_M_BDIRECT;
   if (variant == WAVE_MXFP4_VARIANT_MID_M_BDIRECT) {
-    const bool native = a_scale_layout == WAVE_MXFP4_SCALE_MFMA32 && b_scale_layout == WAVE_MXFP4_SCALE_MFMA32;
-    if (!midb_shape_ok(m, n, k, b_layout) || split_k > 1 || (!native && !workspace)) return WAVE_MXFP4_ERR_UNSUPPORTED;
+    if (!midb_shape_ok(m, n, k, b_layout) || split_k > 1 || (!midb_in_place && !workspace)) return WAVE_MXFP4_ERR_UNSUPPORTED;
   }
   if (variant == WAVE_MXFP4_VARIANT_MID_M) {
     const bool native = (mid_reads(a_scale_layout) || a_scale_layout == WAVE_MXFP4_SCALE_PER_ROW) && mid_reads(b_scale_layout);
@@ -722,7 +726,8 @@ int wave_mxfp4_gemm(const void *a, const void *a_scale, const void *b, const voi
                            asym_gemm_applies(q, device_cus(), false)) ||
                           persist_gemm_applies(q, v, device_cus());
   }
-  if (wants_mfma32_scales(v) && workspace && !small_short && !shuffled_in_place) {
+  if (wants_mfma32_scales(v) && workspace && !small_short && !shuffled_in_place &&
+      !(v == WAVE_MXFP4_VARIANT_MID_M_BDIRECT && both_shuffled)) {
     const size_t a_bytes = round_up_256(scale_buffer_bytes(m, k)), b_bytes = round_up_256(scale_buffer_bytes(n, k));
     const bool mid = v == WAVE_MXFP4_VARIANT_MID_M;
     // (the mid-M kernel reads row-major and e8m0_shuffle scales in place, but only with whole K tiles)

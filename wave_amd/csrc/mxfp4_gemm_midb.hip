@@ -21,8 +21,14 @@
 // One barrier per K tile.  The waits for A are counted (s_waitcnt vmcnt(n)): vector memory operations retire in
 // issue order, and every wave issues the same operations per K tile in a fixed order.
 //
-// Taken for preshuffled B, both scale tensors in MFMA32 order, N % 32 == 0, K a multiple of 1024 (BM = 256) or
-// 2048 (BM = 128): the K loop is unrolled over the ring.  Dense, no split.
+// Taken for preshuffled B, both scale tensors in MFMA32 order or both in e8m0_shuffle order (SHUF: the reference's
+// format for preshuffled operands, read as it is), N % 32 == 0, K a multiple of 1024 (BM = 256) or 2048 (BM = 128):
+// the K loop is unrolled over the ring.  Dense, no split.
+//
+// SHUF: the blocks are the same 256 bytes per 32 rows and K tile, a lane's four bytes sit in two dwords of it, 128
+// bytes apart, joined by one v_perm: two LDS reads per row block for A, two 4-byte requests per K tile for B.  A
+// launch that re-laid both tensors out first cost 8.6 us per call: 256 x 28672 x 8192 50.1 -> 40.7 us (40.2 with the
+// scales in MFMA32 order), 128 rows 27.2 (27.0).
 #include <type_traits>
 
 #include "mxfp4_tile_common.h"
@@ -36,8 +42,9 @@ constexpr int kMidbOnce = 2;   // the "nt" bit: B is read exactly once (M = 128:
 constexpr int kMidbBSets = 4;  // K tiles of B fragments in registers (8 of them: 31.6 us against 29.6)
 constexpr int kMidbDead = (int)0x80000000;  // a scalar offset past the end of any descriptor: nothing is fetched
 
-template <int BM_>
+template <int BM_, bool SHUF_ = false>
 struct MidbCfg {
+  static constexpr bool SHUF = SHUF_;
   static constexpr int BM = BM_, MT = BM / 32;
   static constexpr int SLOT = BM * kTileKBytes;        // 16 / 32 KB of A per K tile
   static constexpr int RING = BM == 256 ? 4 : 8;       // K tiles of A in LDS = K tiles of B in registers = unroll
@@ -47,7 +54,8 @@ struct MidbCfg {
   static constexpr int LDS = RING * SLOT + RING * SSLOT + kMidbWaves * STAGE;
   static constexpr int A_LD = BM / 8 / kMidbWaves;     // A DMA instructions per wave and K tile (4 / 8)
   static constexpr int AS_LD = MT / kMidbWaves;        // A scale DMA instructions per wave and K tile (1 / 2)
-  static constexpr int OPS = A_LD + AS_LD + 4 + 1;     // vector memory operations per wave and K tile
+  static constexpr int BS_LD = SHUF ? 2 : 1;           // B scale requests per wave and K tile
+  static constexpr int OPS = A_LD + AS_LD + 4 + BS_LD;  // vector memory operations per wave and K tile
   // At the wait of K tile j (before its fourth K step) A(j + 1) and its scales must have landed.  They were
   // requested in K tile j + 1 - LA, at the latest as the last operations of its fourth K step, followed by the
   // operations of LA - 2 whole K tiles and those of the first three K steps of K tile j.
@@ -91,6 +99,11 @@ __device__ __forceinline__ void midb_body(const GemmParams &p) {
   const int fr = lane & 31, fg = lane >> 5;
   const int b_goff = wave * 32 * kp + (fr >> 4) * 16 * kp + fg * 256 + (fr & 15) * 16;
   const int s_goff = lane * 4;  // a lane's dword of a 256-byte scale block
+  // e8m0_shuffle order: group g of row r is byte (g % 4) * 64 + (r % 16) * 4 + (g / 4) * 2 + r / 16 of the block; the
+  // dword at sh_goff holds groups fg and 4 + fg, the one 128 bytes on groups 2 + fg and 6 + fg, each for rows r % 16
+  // and r % 16 + 16
+  const int sh_goff = fg * 64 + (fr & 15) * 4;
+  const uint32_t sh_sel = (fr >> 4) ? 0x07030501u : 0x06020400u;
   // A fragment reads: row fr of a 32-row block, chunk 2t + fg at its swizzled position
   uint32_t foff[4];
 #pragma unroll
@@ -118,8 +131,14 @@ __device__ __forceinline__ void midb_body(const GemmParams &p) {
   auto load_b = [&](int kt, int t, v4i &dst, int dead) {
     dst = __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, b_goff, ((kt * 4 + t) * 512) | dead, kMidbOnce);
   };
-  auto load_bs = [&](int kt, uint32_t &dst, int dead) {
-    dst = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(bs_rsrc, s_goff, (wave * k_tiles_blocks + kt * 256) | dead, 0);
+  auto load_bs = [&](int kt, uint32_t (&dst)[Cfg::BS_LD], int dead) {
+    const int so = (wave * k_tiles_blocks + kt * 256) | dead;
+    if constexpr (Cfg::SHUF) {
+      dst[0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(bs_rsrc, sh_goff, so, 0);
+      dst[1] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(bs_rsrc, sh_goff + 128, so, 0);
+    } else {
+      dst[0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(bs_rsrc, s_goff, so, 0);
+    }
   };
 
   // ---------------- registers ----------------
@@ -129,7 +148,7 @@ __device__ __forceinline__ void midb_body(const GemmParams &p) {
 #pragma unroll
     for (int g = 0; g < 16; ++g) acc[i][g] = 0.f;
   v4i bq[kMidbBSets][4];        // [K tile mod sets][K step]
-  uint32_t sb_in[kMidbBSets];   // B scales arriving, per set
+  uint32_t sb_in[kMidbBSets][Cfg::BS_LD];  // B scales arriving, per set
   uint32_t sb_cur;        // ... of the K tile being multiplied
   uint32_t sa[2][MT];     // A scales per parity of the K tile
   v4i afr[2][MT];         // A fragments, double buffered by K step
@@ -140,9 +159,12 @@ __device__ __forceinline__ void midb_body(const GemmParams &p) {
     for (int i = 0; i < MT; ++i) dst[i] = *(const v4i *)(base + i * 32 * kTileKBytes);
   };
   auto read_sa = [&](int slot, uint32_t (&dst)[MT]) {
-    const uint8_t *base = s_ring + slot * Cfg::SSLOT + lane * 4;
+    const uint8_t *base = s_ring + slot * Cfg::SSLOT + (Cfg::SHUF ? sh_goff : s_goff);
 #pragma unroll
-    for (int i = 0; i < MT; ++i) dst[i] = *(const uint32_t *)(base + i * 256);
+    for (int i = 0; i < MT; ++i) {
+      dst[i] = *(const uint32_t *)(base + i * 256);
+      if constexpr (Cfg::SHUF) dst[i] = __builtin_amdgcn_perm(*(const uint32_t *)(base + i * 256 + 128), dst[i], sh_sel);
+    }
   };
   auto mfma_step = [&](const v4i (&fa)[MT], const v4i &fb, const uint32_t (&sca)[MT], uint32_t scb, auto t_tag) {
     constexpr int T = decltype(t_tag)::value;
@@ -180,7 +202,10 @@ __device__ __forceinline__ void midb_body(const GemmParams &p) {
     constexpr int SL_A = (U + LA) % RING, SL_N = (U + 1) % RING;
     // this K tile's B scales were requested four K tiles ago: a real move, pinned here (a compiler copy would be folded
     // into a phi of the loop and wait wherever that lands)
-    asm volatile("v_mov_b32 %0, %1" : "=v"(sb_cur) : "v"(sb_in[SB]));
+    if constexpr (Cfg::SHUF)
+      asm volatile("v_perm_b32 %0, %1, %2, %3" : "=v"(sb_cur) : "v"(sb_in[SB][1]), "v"(sb_in[SB][0]), "v"(sh_sel));
+    else
+      asm volatile("v_mov_b32 %0, %1" : "=v"(sb_cur) : "v"(sb_in[SB][0]));
     read_a(U, 1, afr[1]);
     mfma_step(afr[0], bq[SB][0], sa[PAR], sb_cur, T0{});
     issue_a(ka, SL_A, 0, dead_a);
@@ -355,7 +380,9 @@ int midb_block_rows(const GemmParams &p) {
 // tiles in whole turns of the ring.
 bool midb_gemm_applies(const GemmParams &p) {
   if (!p.b_preshuffled || p.num_groups != 0 || p.tile_table != nullptr || p.splits != 1 || p.partial != nullptr) return false;
-  if (p.a_scale_layout != WAVE_MXFP4_SCALE_MFMA32 || p.b_scale_layout != WAVE_MXFP4_SCALE_MFMA32) return false;
+  if (p.a_scale_layout != p.b_scale_layout ||
+      (p.a_scale_layout != WAVE_MXFP4_SCALE_MFMA32 && p.a_scale_layout != WAVE_MXFP4_SCALE_E8M0_SHUFFLE))
+    return false;
   if ((p.n & 31) != 0 || (p.k & (kTileK - 1)) != 0 || p.k_tiles * 256 != p.k) return false;
   if (midb_block_rows(p) == 0) return false;
   // 32-bit offsets: a strip of B, all of A, all of C
@@ -366,9 +393,13 @@ bool midb_gemm_applies(const GemmParams &p) {
 }
 
 hipError_t launch_midb_gemm(const GemmParams &p, hipStream_t stream) {
-  if (midb_block_rows(p) == 128)
-    return p.out_bf16 ? launch_midb_out<MidbCfg<128>, true>(p, stream) : launch_midb_out<MidbCfg<128>, false>(p, stream);
-  return p.out_bf16 ? launch_midb_out<MidbCfg<256>, true>(p, stream) : launch_midb_out<MidbCfg<256>, false>(p, stream);
+  const bool shuf = p.a_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE;
+  const auto launch = [&](auto plain, auto shuffled) {
+    if (shuf)
+      return p.out_bf16 ? launch_midb_out<decltype(shuffled), true>(p, stream) : launch_midb_out<decltype(shuffled), false>(p, stream);
+    return p.out_bf16 ? launch_midb_out<decltype(plain), true>(p, stream) : launch_midb_out<decltype(plain), false>(p, stream);
+  };
+  return midb_block_rows(p) == 128 ? launch(MidbCfg<128>{}, MidbCfg<128, true>{}) : launch(MidbCfg<256>{}, MidbCfg<256, true>{});
 }
 
 }  // namespace wave_mxfp4
