@@ -5,10 +5,13 @@ does not load, every operator of this package raises."""
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # WAVE_MXFP4_LIB points at another build of the same ABI (e.g. an experiment)
+HOST_PATH = os.path.join(_HERE, "csrc", "_wave_host.so")
 LIB_PATH = os.environ.get("WAVE_MXFP4_LIB") or os.path.join(_HERE, "csrc", "libwave_mxfp4.so")
 
 ABI_VERSION = 10
@@ -75,6 +78,25 @@ EXPORTS = (
 )
 
 _lib = None
+host = None  # the native call path (csrc/wave_host.cpp), set by load_host()
+
+
+def load_host():
+    """Import the native call path and hand it the entry points of the library :func:`load` opened."""
+    global host
+    lib = load()
+    if host is None:
+        import torch  # noqa: F401  (the module's symbols come from torch's libraries)
+
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `make -C {os.path.dirname(HOST_PATH)}`")
+        loader = importlib.machinery.ExtensionFileLoader("_wave_host", HOST_PATH)
+        spec = importlib.util.spec_from_file_location("_wave_host", HOST_PATH, loader=loader)
+        mod = importlib.util.module_from_spec(spec)
+        loader.exec_module(mod)
+        mod.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in EXPORTS})
+        host = mod
+    return host
 
 
 def load():
