@@ -13,8 +13,34 @@ namespace {
 
 constexpr int kAlignWaves = 16;
 constexpr int kAlignThreads = kAlignWaves * 64;
-constexpr int kFewExperts = 16;
+// Steps of 64 entries whose places a wave keeps in registers between the count and the placement: 16 steps x 16
+// waves = 16384 entries, read and ranked once.  A longer table is ranked a second time when it is placed.
+constexpr int kRegSteps = 16;
 
+// The place of every lane's entry among the entries of its expert that the wave has met so far, and the count of them
+// moved on: `row[e]` before this step plus the lanes of the same expert below this one.  The lanes of one expert are
+// found with one ballot per bit of the id (`bits` of them) and not with a turn per expert that occurs, which left a
+// chain of 28 dependent turns per 64 entries at 32 experts.  The wave's LDS operations complete in their order, so
+// the steps need no wait in between: the leader's addition follows every lane's read, the next step's read follows it.
+__device__ __forceinline__ int rank_in_expert(int e, bool valid, int bits, int lane, int *row) {
+  uint64_t same = __ballot(valid);
+  for (int b = 0; b < bits; ++b) {
+    const bool one = (e >> b) & 1;
+    const uint64_t ones = __ballot(one);
+    same &= one ? ones : ~ones;
+  }
+  const int below = __popcll(same & ((1ull << lane) - 1));
+  int before = 0;
+  if (valid) before = __hip_atomic_load(row + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (valid && below == 0)
+    __hip_atomic_fetch_add(row + e, __popcll(same), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  return before + below;
+}
+
+// Bound by latency: one round trip for the ids, the ranks of a wave's steps (about 45 vector instructions per 64
+// entries at 32 experts), two barriers, one store.  MI355X, a whole expert MLP with it (us, a turn per expert that
+// occurs -> ballots): 8452 entries of 32 experts 417 -> 374 (the kernel alone took 59 of them), 3672 of 32 207 -> 188,
+// 192 of 32 128.4 -> 124.8, 8192 of 8 experts 810 -> 808.
 template <typename IdT>
 __global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(const IdT *__restrict__ topk_ids, int n, int num_experts,
                                                                   int block_size, int32_t *__restrict__ sorted_ids,
@@ -23,34 +49,40 @@ __global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(const IdT *__r
                                                                   int32_t *__restrict__ offsets_out) {
   extern __shared__ int lds[];
   int *cnt = lds;                                // [kAlignWaves][E]: entries of expert e in wave w's segment, later
-                                                 // the next free position for them
+                                                 // the first (a long table: the next) position for them
   int *wave_sums = lds + kAlignWaves * num_experts;  // [kAlignWaves]
   int *starts = wave_sums + kAlignWaves;             // [E + 1]: first position of every expert's run, then the total
   int *counts = starts + num_experts + 1;            // [E]: entries of every expert
   const int E = num_experts;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-
-  for (int i = t; i < kAlignWaves * E; i += kAlignThreads) cnt[i] = 0;
-  __syncthreads();
+  const int bits = E > 1 ? 32 - __clz(E - 1) : 0;
+  int *row = cnt + wave * E;
 
   // wave w owns the contiguous segment [seg0, seg1) of the flat table
   const int per_wave = ((n + kAlignWaves - 1) / kAlignWaves + 63) & ~63;
   const int seg0 = min(n, wave * per_wave), seg1 = min(n, seg0 + per_wave);
-  // (8 steps of 64 ids are fetched together: a step at a time would pay a memory round trip each; the first
-  // eight steps stay in registers for the placement below: up to 8192 entries are read once)
-  int64_t e_first[8];
-  for (int base = seg0; base < seg1; base += 8 * 64) {
-    int64_t e[8];
+  const bool in_regs = per_wave <= kRegSteps * 64;
+
+  // (all steps' ids are fetched together: a step at a time would pay a memory round trip each)
+  int id[kRegSteps], place[kRegSteps];
+  auto fetch = [&](int base) {
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
+    for (int s = 0; s < kRegSteps; ++s) {
       const int i = base + s * 64 + lane;
-      e[s] = i < seg1 ? (int64_t)topk_ids[i] : -1;
-      if (base == seg0) e_first[s] = e[s];
+      const int64_t v = i < seg1 ? (int64_t)topk_ids[i] : -1;
+      id[s] = v >= 0 && v < E ? (int)v : -1;
     }
+  };
+  auto rank = [&](int base) {
 #pragma unroll
-    for (int s = 0; s < 8; ++s)
-      if (e[s] >= 0 && e[s] < E) atomicAdd(&cnt[wave * E + (int)e[s]], 1);
-  }
+    for (int s = 0; s < kRegSteps; ++s)
+      if (base + s * 64 < seg1) place[s] = rank_in_expert(id[s], id[s] >= 0, bits, lane, row);
+  };
+  fetch(seg0);
+  for (int i = t; i < kAlignWaves * E; i += kAlignThreads) cnt[i] = 0;
+  __syncthreads();
+  rank(seg0);
+  for (int base = seg0 + kRegSteps * 64; base < seg1; base += kRegSteps * 64) fetch(base), rank(base);
   __syncthreads();
 
   // thread e: the expert's count, padded count and first position
@@ -74,6 +106,25 @@ __global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(const IdT *__r
   }
   if (t == kAlignThreads - 1) starts[E] = end;
   __syncthreads();
+
+  // place
+  if (in_regs) {
+#pragma unroll
+    for (int s = 0; s < kRegSteps; ++s)
+      if (id[s] >= 0) {
+        const int pos = row[id[s]] + place[s];
+        if (pos < sorted_len) sorted_ids[pos] = seg0 + s * 64 + lane;
+      }
+  } else {
+    for (int base = seg0; base < seg1; base += kRegSteps * 64) {
+      fetch(base);
+      rank(base);
+#pragma unroll
+      for (int s = 0; s < kRegSteps; ++s)
+        if (id[s] >= 0 && place[s] < sorted_len) sorted_ids[place[s]] = base + s * 64 + lane;
+    }
+  }
+
   const int total = starts[E];
   if (t == 0) {
     total_out[0] = total;
@@ -89,61 +140,6 @@ __global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(const IdT *__r
   for (int e = wave; e < E; e += kAlignWaves) {
     const int from = starts[e] / block_size, to = min(starts[e + 1] / block_size, expert_ids_len);
     for (int b = from + lane; b < to; b += 64) expert_ids[b] = e;
-  }
-
-  // place: a wave walks its segment in order; the lanes of one expert take consecutive positions
-  // Up to 64 experts the wave keeps "next free position of expert e" in lane e's register (a readlane per
-  // look-up); beyond that in its row of cnt (an LDS round trip per look-up).
-  const bool in_regs = E <= 64;
-  volatile int *next = cnt + wave * E;
-  int next_reg = in_regs && lane < E ? cnt[wave * E + lane] : 0;
-  for (int base8 = seg0; base8 < seg1; base8 += 8 * 64) {
-    int64_t e8[8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int i = base8 + s * 64 + lane;
-      e8[s] = base8 == seg0 ? e_first[s] : i < seg1 ? (int64_t)topk_ids[i] : -1;
-    }
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int i = base8 + s * 64 + lane;
-      const bool valid = e8[s] >= 0 && e8[s] < E;
-      const int e = valid ? (int)e8[s] : -1;
-      if (__ballot(valid) == 0) continue;  // (a short table: most of the eight steps hold no entry at all)
-      if (E <= kFewExperts) {
-        // few experts: one ballot per expert, no search for the experts that occur
-        int pos = -1;
-#pragma unroll
-        for (int x = 0; x < kFewExperts; ++x) {
-          if (x < E) {
-            const uint64_t same = __ballot(e == x);
-            const int first = __builtin_amdgcn_readlane(next_reg, x);
-            if (e == x) pos = first + __popcll(same & ((1ull << lane) - 1));
-            if (lane == x) next_reg += __popcll(same);
-          }
-        }
-        if (pos >= 0 && pos < sorted_len) sorted_ids[pos] = i;
-        continue;
-      }
-      uint64_t todo = __ballot(valid);
-      while (todo) {
-        const int leader = __ffsll((unsigned long long)todo) - 1;
-        const int e0 = __builtin_amdgcn_readlane(e, leader);
-        const uint64_t same = __ballot(e == e0);
-        const int first = in_regs ? __builtin_amdgcn_readlane(next_reg, e0) : next[e0];
-        if (e == e0) {
-          const int pos = first + __popcll(same & ((1ull << lane) - 1));
-          if (pos < sorted_len) sorted_ids[pos] = i;
-        }
-        const int taken = __popcll(same);
-        if (in_regs) {
-          if (lane == e0) next_reg += taken;
-        } else if (lane == leader) {
-          next[e0] = first + taken;
-        }
-        todo &= ~same;
-      }
-    }
   }
 }
 
