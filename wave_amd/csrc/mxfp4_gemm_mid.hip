@@ -54,10 +54,17 @@ constexpr int kMidOnce = 2;  // the "nt" bit: B is read exactly once
 // 6.75 TB/s); with one workgroup per CU or fewer the deep rings are the better use of the LDS.
 // A_OFF: A's scales are in MFMA32 order and the block of rows may start inside one of their 32-row blocks (a group
 // of a grouped problem starts at any row): the images hold one block more.
-template <int BM_, bool B_RM_, bool TWO_PER_CU_ = false, bool A_OFF_ = false>
+// B_KEEP: B's requests without the "nt" bit.  Rows of B that are not whole 128-byte lines (K % 256 != 0) share lines
+// between neighbouring K tiles and neighbouring rows: every 128-byte piece of a row touches two lines, and with the
+// bit the half that the next K tile needs is dropped before it asks (an expert MLP of 32 experts x 2880 x 2880, us,
+// with the bit -> without: 192 rows 124.8 -> 112.4, 1200 rows 145.9 -> 131.8, 3672 rows 188.5 -> 176.4; whole
+// lines lose without it: 16 experts x 4096 x 4096, 96 rows 80.2 -> 90.6, 8 x 14336 x 4096, 128 rows 130 -> 149).  The
+// 256-row block keeps the bit: its A, re-read by every workgroup, is what L2 must hold (256 x 24576 x 5728 39.6 -> 41.0).
+template <int BM_, bool B_RM_, bool TWO_PER_CU_ = false, bool A_OFF_ = false, bool B_KEEP_ = false>
 struct MidCfg {
   static constexpr int BM = BM_, MT_M = BM / 32;
   static constexpr bool B_RM = B_RM_, TWO_PER_CU = TWO_PER_CU_, A_OFF = A_OFF_;
+  static constexpr bool B_KEEP = B_KEEP_;
   static_assert(!TWO_PER_CU || BM == 32, "only the 32-row block leaves room for two workgroups");
   // The four compute waves sit WM x (4 / WM) on the strip: two row halves times two pairs of column groups from
   // BM = 64 on (one A fragment per two MFMAs), side by side on one row block at BM = 32.
@@ -228,9 +235,13 @@ __device__ __forceinline__ void mid_body(const GemmParams &p, const int wv, cons
   auto issue_b = [&](int v, int slot) {
     const int soff = v < vend ? tile_of(v) * b_kt_stride : (int)0x80000000;
 #pragma unroll
-    for (int d = 0; d < 4; ++d)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, WAVE_LDS_PTR(b_ring + slot * 16384 + wave * 4096 + d * 1024), 16,
-                                               b_goff[d], soff, 0, kMidOnce);
+    for (int d = 0; d < 4; ++d) {
+      uint8_t *dst = b_ring + slot * 16384 + wave * 4096 + d * 1024;
+      if constexpr (Cfg::B_KEEP)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, WAVE_LDS_PTR(dst), 16, b_goff[d], soff, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, WAVE_LDS_PTR(dst), 16, b_goff[d], soff, 0, kMidOnce);
+    }
   };
   // MFMA32 order: the four 256-byte blocks of K tiles 4g .. 4g + 3 are contiguous, one instruction per group.
   auto issue_bs = [&](int g) {
@@ -620,6 +631,12 @@ hipError_t launch_mid_layouts(const GemmParams &p, int wv, hipStream_t stream) {
 template <int BM, bool TWO = false>
 hipError_t launch_mid_cfg(const GemmParams &p, int wv, hipStream_t stream) {
   const bool a_rm = p.a_scale_layout == WAVE_MXFP4_SCALE_ROW_MAJOR, b_rm = p.b_scale_layout == WAVE_MXFP4_SCALE_ROW_MAJOR;
+  if constexpr (BM <= 192) {
+    // rows of B that are not whole lines (both scale tensors are in MFMA32 order then: mid_gemm_applies)
+    if ((p.kp & (kTileKBytes - 1)) != 0 && !p.b_preshuffled)
+      return p.num_groups == 0 ? launch_mid_kernel<MidCfg<BM, false, TWO, false, true>, false, false, false>(p, wv, stream)
+                               : launch_mid_kernel<MidCfg<BM, false, TWO, true, true>, false, true, false>(p, wv, stream);
+  }
   if (p.num_groups != 0) {  // (A's scales row-major or MFMA32: checked by mid_grouped_applies)
     if constexpr (BM <= 192) {
       if (!a_rm)
