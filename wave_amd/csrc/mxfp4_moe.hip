@@ -65,24 +65,22 @@ __global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(const IdT *__r
 
   // (all steps' ids are fetched together: a step at a time would pay a memory round trip each)
   int id[kRegSteps], place[kRegSteps];
-  auto fetch = [&](int base) {
+  auto fetch_and_rank = [&](int base) {
 #pragma unroll
     for (int s = 0; s < kRegSteps; ++s) {
+      id[s] = -1;
+      if (base + s * 64 >= seg1) continue;
       const int i = base + s * 64 + lane;
       const int64_t v = i < seg1 ? (int64_t)topk_ids[i] : -1;
       id[s] = v >= 0 && v < E ? (int)v : -1;
     }
-  };
-  auto rank = [&](int base) {
 #pragma unroll
     for (int s = 0; s < kRegSteps; ++s)
       if (base + s * 64 < seg1) place[s] = rank_in_expert(id[s], id[s] >= 0, bits, lane, row);
   };
-  fetch(seg0);
   for (int i = t; i < kAlignWaves * E; i += kAlignThreads) cnt[i] = 0;
   __syncthreads();
-  rank(seg0);
-  for (int base = seg0 + kRegSteps * 64; base < seg1; base += kRegSteps * 64) fetch(base), rank(base);
+  for (int base = seg0; base < seg1; base += kRegSteps * 64) fetch_and_rank(base);
   __syncthreads();
 
   // thread e: the expert's count, padded count and first position
@@ -110,15 +108,16 @@ __global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(const IdT *__r
   // place
   if (in_regs) {
 #pragma unroll
-    for (int s = 0; s < kRegSteps; ++s)
+    for (int s = 0; s < kRegSteps; ++s) {
+      if (seg0 + s * 64 >= seg1) break;
       if (id[s] >= 0) {
         const int pos = row[id[s]] + place[s];
         if (pos < sorted_len) sorted_ids[pos] = seg0 + s * 64 + lane;
       }
+    }
   } else {
     for (int base = seg0; base < seg1; base += kRegSteps * 64) {
-      fetch(base);
-      rank(base);
+      fetch_and_rank(base);
 #pragma unroll
       for (int s = 0; s < kRegSteps; ++s)
         if (id[s] >= 0 && place[s] < sorted_len) sorted_ids[place[s]] = base + s * 64 + lane;
