@@ -496,6 +496,132 @@ bool split_ok(int64_t k, int splits, int *tiles_per_split) {
   return true;
 }
 
+// Bytes of one operand's scales in the padded non row-major layouts.
+size_t scale_buffer_bytes(int64_t rows, int64_t k) {
+  const int64_t ks = k / 32;
+  return (size_t)((rows + 31) / 32 * 32) * (size_t)((ks + 7) / 8 * 8);
+}
+size_t round_up_256(size_t v) { return (v + 255) / 256 * 256; }
+
+// ---- The deep-ring kernel (mxfp4_gemm_deep.hip): the tile shape and the parts along K for a dense problem ----
+// It runs one workgroup per CU, so it is for problems that are one round of its tiles at most.  Which shape and how many
+// parts is an estimate (us) from the same quantities as above, fitted to 300 random shapes (M = 1 .. 4096, N = 1024 ..
+// 28672, K = 1024 .. 16384, weights from HBM, every shape with 1-8 parts by name: the choice is at 1.0135 of the best
+// of them in the geometric mean): a fixed part, a workgroup's time per K tile at 0 / 64 / 128 / 192 / 256 workgroups in
+// flight, a split's reduction, and what row-major scales cost when the workgroups stage them themselves (`rows`, up
+// to rows_max K tiles each) or when a launch in front re-lays them.
+struct DeepShape {
+  int bm, bn, rows_max;
+  double fixed, step[5], split, rows_step, rows;
+};
+constexpr DeepShape kDeepShapes[] = {
+    {64, 64, 15, 3.81, {0.212, 0.246, 0.275, 0.306, 0.364}, 2.30, 0.557, 0.0},
+    {64, 128, 9, 3.94, {0.308, 0.424, 0.489, 0.571, 0.674}, 2.43, 0.217, 0.2},
+    {128, 128, 15, 3.63, {0.339, 0.469, 0.566, 0.613, 0.822}, 2.50, 0.365, 0.2},
+    {128, 256, 5, 4.70, {0.503, 0.803, 0.926, 1.002, 1.392}, 2.04, 0.112, 0.6},
+    {256, 128, 5, 5.00, {0.440, 0.618, 0.739, 0.795, 1.268}, 2.13, 0.249, 0.4},
+};
+struct DeepChoice {
+  int shape = -1, splits = 1;
+  bool relayout = false;  // both scale tensors go through scratch into MFMA32 order
+  size_t bytes = 0;       // scratch: the parts, then the re-laid scales
+};
+enum DeepScaleMode { kDeepNone, kDeepBlocked, kDeepRowMajor };
+
+DeepScaleMode deep_scale_mode(int64_t k, int asl, int bsl) {
+  if (asl != bsl) return kDeepNone;
+  if (asl == WAVE_MXFP4_SCALE_MFMA32) return kDeepBlocked;  // (a partial last K tile: mxfp4_gemm_deep.hip)
+  if (asl == WAVE_MXFP4_SCALE_E8M0_SHUFFLE) return k % kTileK == 0 ? kDeepBlocked : kDeepNone;
+  return asl == WAVE_MXFP4_SCALE_ROW_MAJOR ? kDeepRowMajor : kDeepNone;
+}
+
+// Whether the deep-ring kernel takes the problem from kernel `v`.  Measured borders (us, `v` -> deep):
+//   scales in a blocked order.  More than 128 rows: always (387 x 2048 x 4096 15.8 -> 8.1, 1000 x 7168 x 4096 24.5 -> 21.3,
+//     2048 x 4096 x 14336 68.4 -> 59.6).  17 .. 128 rows up to N = 16384 (128 x 3840 x 4096 13.5 -> 8.0, 38 x 13568 x
+//     5632 13.6 -> 11.5; 36 x 17152 x 8448 loses to the mid-M kernel, 19.6 -> 21.1).  Up to 16 rows the streaming kernel
+//     keeps the K ranges that it runs with counted waits (12 x 3104 x 6144 7.1, here 8.5) and narrow B of 12 .. 32 K
+//     tiles (3 x 1280 x 6400 6.6, here 7.9); the rest is taken: 1 x 5632 x 1024 8.2 -> 4.8, 2 x 3200 x 13568 14.0 ->
+//     10.2, 1 x 4096 x 6080 16.5 -> 8.6, 2 x 11424 x 5920 18.2 -> 11.1.
+//   row-major scales.  From a tile kernel: always (192 x 4608 x 2304 13.5 -> 7.5, 727 x 4096 x 11008 43.4 -> 34.1).  The
+//     streaming and the mid-M kernel read them in place, so there only a narrow B and no launch in front (62 x 3104 x
+//     1280 10.9 -> 5.8, 128 x 6144 x 8960 20.5 -> 18.2; 147 x 8544 x 3072 loses, 12.8 -> 14.1), and up to 16 rows only
+//     up to 6 K tiles or beyond the streaming kernel's 32 (4 x 1792 x 13824 14.9 -> 9.9; 3 x 4096 x 5632 loses, 7.0 -> 9.3).
+bool deep_over(int v, int64_t m, int64_t n, int64_t k, DeepScaleMode mode, bool *no_relayout) {
+  *no_relayout = false;
+  if (v == WAVE_MXFP4_VARIANT_MID_M_BDIRECT || v == WAVE_MXFP4_VARIANT_NAIVE) return false;
+  const int64_t kt = (k + kTileK - 1) / kTileK;
+  if (mode == kDeepRowMajor) {
+    if (is_tile_variant(v)) return true;
+    *no_relayout = true;
+    return n <= 6144 && k % kTileK == 0 && (m > 16 || kt <= 6 || kt > 32);
+  }
+  if (m > 128) return true;
+  if (n > 16384) return false;
+  if (m > 16 || kt <= 11) return true;
+  if (kt <= 32) return n >= 4096 && !stream_runs_counted(n, k);
+  return n <= 8192 || !stream_runs_counted(n, k);
+}
+
+// The cheapest shape and split within `room` bytes of scratch; shape < 0: not for this kernel.
+DeepChoice deep_choice(int v, int64_t m, int64_t n, int64_t k, int out_dtype, int asl, int bsl, size_t room) {
+  DeepChoice best;
+  const DeepScaleMode mode = deep_scale_mode(k, asl, bsl);
+  bool no_relayout = false;
+  if (mode == kDeepNone || n < 1024 || k < 1024 || n % (out_dtype == WAVE_MXFP4_OUT_BF16 ? 8 : 4) != 0 ||
+      !deep_over(v, m, n, k, mode, &no_relayout))
+    return best;
+  const int64_t kt = (k + kTileK - 1) / kTileK;
+  const double scale_cus = 256.0 / (double)device_cus();
+  double best_us = 1e30;
+  for (int i = 0; i < (int)(sizeof(kDeepShapes) / sizeof(kDeepShapes[0])); ++i) {
+    const DeepShape &d = kDeepShapes[i];
+    const int64_t tiles = ((m + d.bm - 1) / d.bm) * ((n + d.bn - 1) / d.bn);
+    for (int s = 1; s <= 8 && tiles * s <= device_cus(); ++s) {
+      const int64_t per = (kt + s - 1) / s;
+      if (s > 1 && (kt / s < 2 || (s - 1) * per >= kt)) continue;
+      const bool rows = mode == kDeepRowMajor && k % kTileK == 0 && per <= d.rows_max;
+      const bool relayout = mode == kDeepRowMajor && !rows;
+      if (relayout && no_relayout) continue;
+      const size_t parts = s > 1 ? round_up_256((size_t)s * (size_t)m * (size_t)n * sizeof(float)) : 0;
+      const size_t bytes =
+          parts + (relayout ? round_up_256(scale_buffer_bytes(m, k)) + round_up_256(scale_buffer_bytes(n, k)) : 0);
+      if (bytes > room) continue;
+      const double w = (double)(tiles * s) * scale_cus / 64.0;
+      const int at = w >= 4.0 ? 3 : (int)w;
+      double us = d.fixed + (double)per * (d.step[at] + (w - at) * (d.step[at + 1] - d.step[at])) * (rows ? 1.0 + d.rows_step : 1.0);
+      if (rows) us += d.rows;
+      if (relayout) us += 4.5 + (double)(n * k) / 80.0e6;
+      if (s > 1) us += d.split + 0.05 * s + 1.3e-6 * (double)s * (double)m * (double)n;
+      if (us < best_us) {
+        best_us = us;
+        best.shape = i, best.splits = s, best.relayout = relayout, best.bytes = bytes;
+      }
+    }
+  }
+  return best;
+}
+
+hipError_t run_deep(GemmParams p, const DeepChoice &d, void *workspace, hipStream_t stream) {
+  uint8_t *ws = (uint8_t *)workspace;
+  hipError_t e;
+  if (d.splits > 1) {
+    p.splits = d.splits;
+    p.tiles_per_split = (p.k_tiles + d.splits - 1) / d.splits;
+    p.partial = (float *)ws;
+    ws += round_up_256((size_t)d.splits * (size_t)p.m * (size_t)p.n * sizeof(float));
+  }
+  if (d.relayout) {
+    uint8_t *bs = ws + round_up_256(scale_buffer_bytes(p.m, p.k));
+    e = launch_scale_pair_to_mfma32(p.a_scale, ws, p.m, p.b_scale, bs, p.n, p.ks, stream);
+    if (e != hipSuccess) return e;
+    p.a_scale = ws, p.b_scale = bs;
+    p.a_scale_layout = p.b_scale_layout = WAVE_MXFP4_SCALE_MFMA32;
+  }
+  e = launch_deep_gemm(p, d.shape, stream);
+  if (e != hipSuccess || d.splits == 1) return e;
+  return launch_splitk_reduce(p.partial, p.c, (int64_t)p.m * p.n, d.splits, p.out_bf16, stream);
+}
+
 // Scratch of wave_mxfp4_gemm_static: a fixed array in the library's device image, one copy per GPU, held until
 // the process ends.  On the host the array's name is only a handle for hipGetSymbolAddress: the address a
 // kernel can use is looked up once per device and kept here.
@@ -542,13 +668,6 @@ const char *wave_mxfp4_status_string(int status) {
 
 const char *wave_mxfp4_last_hip_error(void) { return g_hip_error; }
 
-// Bytes of one operand's scales in the padded non row-major layouts.
-static size_t scale_buffer_bytes(int64_t rows, int64_t k) {
-  const int64_t ks = k / 32;
-  return (size_t)((rows + 31) / 32 * 32) * (size_t)((ks + 7) / 8 * 8);
-}
-static size_t round_up_256(size_t v) { return (v + 255) / 256 * 256; }
-
 static size_t workspace_bytes_of(int64_t m, int64_t n, int64_t k, int split_k, int v, bool native_scales) {
   size_t bytes = round_up_256((size_t)m * (size_t)(k / 32));  // per-row A scales spread out to [M, K/32]
   if (v == WAVE_MXFP4_VARIANT_NAIVE) return bytes;
@@ -575,7 +694,16 @@ size_t wave_mxfp4_workspace_bytes(int64_t m, int64_t n, int64_t k, int split_k, 
   // the library's own choice of kernel depends on the scale layouts of the call: the larger of the two
   const size_t plain = workspace_bytes_of(m, n, k, split_k, pick_variant(m, n, k, variant, false, false), false);
   const size_t native = workspace_bytes_of(m, n, k, split_k, pick_variant(m, n, k, variant, true, false), true);
-  return plain > native ? plain : native;
+  size_t most = plain > native ? plain : native;
+  if (variant == WAVE_MXFP4_VARIANT_AUTO && split_k == 0) {
+    for (const int layout : {WAVE_MXFP4_SCALE_ROW_MAJOR, WAVE_MXFP4_SCALE_E8M0_SHUFFLE, WAVE_MXFP4_SCALE_MFMA32}) {
+      const bool nat = layout == WAVE_MXFP4_SCALE_MFMA32;
+      const size_t deep = deep_choice(pick_variant(m, n, k, variant, nat, false), m, n, k, WAVE_MXFP4_OUT_F32, layout,
+                                      layout, SIZE_MAX).bytes;
+      if (deep > most) most = deep;
+    }
+  }
+  return most;
 }
 
 int wave_mxfp4_gemm(const void *a, const void *a_scale, const void *b, const void *b_scale, void *c,
@@ -616,6 +744,11 @@ int wave_mxfp4_gemm(const void *a, const void *a_scale, const void *b, const voi
       (m > 128 ? n <= cus_n
                : midb_in_place && n <= 2 * cus_n && (m >= 64 || (m >= 32 && n <= cus_n && (n >= 20480 || k <= 4096)))))
     v = WAVE_MXFP4_VARIANT_MID_M_BDIRECT;
+  if (variant == WAVE_MXFP4_VARIANT_AUTO && split_k == 0 && k > 0 && (!workspace || aligned(workspace, 256))) {
+    const DeepChoice d =
+        deep_choice(v, m, n, k, out_dtype, a_scale_layout, b_scale_layout, workspace ? workspace_bytes : 0);
+    if (d.shape >= 0) return record_hip(run_deep(p, d, workspace, stream));
+  }
   if (variant == WAVE_MXFP4_VARIANT_MID_M_BDIRECT) {
     if (!midb_shape_ok(m, n, k, b_layout) || split_k > 1 || (!midb_in_place && !workspace)) return WAVE_MXFP4_ERR_UNSUPPORTED;
   }
