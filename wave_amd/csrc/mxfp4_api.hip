@@ -511,15 +511,15 @@ size_t round_up_256(size_t v) { return (v + 255) / 256 * 256; }
 // flight, a split's reduction, and what row-major scales cost when the workgroups stage them themselves (`rows`, up
 // to rows_max K tiles each) or when a launch in front re-lays them.
 struct DeepShape {
-  int bm, bn, rows_max;
+  int index, bm, bn, rows_max;  // index: launch_deep_gemm's shape
   double fixed, step[5], split, rows_step, rows;
 };
 constexpr DeepShape kDeepShapes[] = {
-    {64, 64, 15, 3.81, {0.212, 0.246, 0.275, 0.306, 0.364}, 2.30, 0.557, 0.0},
-    {64, 128, 9, 3.94, {0.308, 0.424, 0.489, 0.571, 0.674}, 2.43, 0.217, 0.2},
-    {128, 128, 15, 3.63, {0.339, 0.469, 0.566, 0.613, 0.822}, 2.50, 0.365, 0.2},
-    {128, 256, 5, 4.70, {0.503, 0.803, 0.926, 1.002, 1.392}, 2.04, 0.112, 0.6},
-    {256, 128, 5, 5.00, {0.440, 0.618, 0.739, 0.795, 1.268}, 2.13, 0.249, 0.4},
+    {0, 64, 64, 15, 3.81, {0.212, 0.246, 0.275, 0.306, 0.364}, 2.30, 0.557, 0.0},
+    {1, 64, 128, 9, 3.94, {0.308, 0.424, 0.489, 0.571, 0.674}, 2.43, 0.217, 0.2},
+    {2, 128, 128, 15, 3.63, {0.339, 0.469, 0.566, 0.613, 0.822}, 2.50, 0.365, 0.2},
+    {3, 128, 256, 5, 4.70, {0.503, 0.803, 0.926, 1.002, 1.392}, 2.04, 0.112, 0.6},
+    {4, 256, 128, 5, 5.00, {0.440, 0.618, 0.739, 0.795, 1.268}, 2.13, 0.249, 0.4},
 };
 struct DeepChoice {
   int shape = -1, splits = 1;
@@ -542,13 +542,17 @@ DeepScaleMode deep_scale_mode(int64_t k, int asl, int bsl) {
 //     keeps the K ranges that it runs with counted waits (12 x 3104 x 6144 7.1, here 8.5) and narrow B of 12 .. 32 K
 //     tiles (3 x 1280 x 6400 6.6, here 7.9); the rest is taken: 1 x 5632 x 1024 8.2 -> 4.8, 2 x 3200 x 13568 14.0 ->
 //     10.2, 1 x 4096 x 6080 16.5 -> 8.6, 2 x 11424 x 5920 18.2 -> 11.1.
+//   the B-direct mid-M kernel keeps a preshuffled B that is wide or meets 65 .. 128 rows (256 x 28672 x 8192 41.7, here
+//     44.3; 128 x 12288 x 4096 12.9, here 14.0; 254 x 15872 x 12288 50.4 -> 42.6, 256 x 12288 x 4096 18.9 -> 16.0,
+//     48 x 12288 x 8192 18.0 -> 16.2; measured from K = 4096 on).
 //   row-major scales.  From a tile kernel: always (192 x 4608 x 2304 13.5 -> 7.5, 727 x 4096 x 11008 43.4 -> 34.1).  The
 //     streaming and the mid-M kernel read them in place, so there only a narrow B and no launch in front (62 x 3104 x
 //     1280 10.9 -> 5.8, 128 x 6144 x 8960 20.5 -> 18.2; 147 x 8544 x 3072 loses, 12.8 -> 14.1), and up to 16 rows only
 //     up to 6 K tiles or beyond the streaming kernel's 32 (4 x 1792 x 13824 14.9 -> 9.9; 3 x 4096 x 5632 loses, 7.0 -> 9.3).
 bool deep_over(int v, int64_t m, int64_t n, int64_t k, DeepScaleMode mode, bool *no_relayout) {
   *no_relayout = false;
-  if (v == WAVE_MXFP4_VARIANT_MID_M_BDIRECT || v == WAVE_MXFP4_VARIANT_NAIVE) return false;
+  if (v == WAVE_MXFP4_VARIANT_NAIVE) return false;
+  if (v == WAVE_MXFP4_VARIANT_MID_M_BDIRECT) return mode == kDeepBlocked && n <= 16384 && k >= 4096 && (m > 128 || m <= 64);
   const int64_t kt = (k + kTileK - 1) / kTileK;
   if (mode == kDeepRowMajor) {
     if (is_tile_variant(v)) return true;
@@ -562,46 +566,73 @@ bool deep_over(int v, int64_t m, int64_t n, int64_t k, DeepScaleMode mode, bool 
   return n <= 8192 || !stream_runs_counted(n, k);
 }
 
-// The cheapest shape and split within `room` bytes of scratch; shape < 0: not for this kernel.
-DeepChoice deep_choice(int v, int64_t m, int64_t n, int64_t k, int out_dtype, int asl, int bsl, size_t room) {
+// The cheapest shape and split of `shapes` within `room` bytes of scratch.  kt: K tiles; rows_ok / relayout_ok: row-major
+// scales may be staged by the workgroups / re-laid by a launch in front (blocked scales need neither: `blocked`).
+DeepChoice deep_search(const DeepShape *shapes, int count, int64_t m, int64_t n, int64_t k, int64_t kt, int min_part,
+                       bool blocked, bool rows_ok, bool relayout_ok, bool four_bit, size_t room) {
   DeepChoice best;
-  const DeepScaleMode mode = deep_scale_mode(k, asl, bsl);
-  bool no_relayout = false;
-  if (mode == kDeepNone || n < 1024 || k < 1024 || n % (out_dtype == WAVE_MXFP4_OUT_BF16 ? 8 : 4) != 0 ||
-      !deep_over(v, m, n, k, mode, &no_relayout))
-    return best;
-  const int64_t kt = (k + kTileK - 1) / kTileK;
   const double scale_cus = 256.0 / (double)device_cus();
   double best_us = 1e30;
-  for (int i = 0; i < (int)(sizeof(kDeepShapes) / sizeof(kDeepShapes[0])); ++i) {
-    const DeepShape &d = kDeepShapes[i];
+  for (int i = 0; i < count; ++i) {
+    const DeepShape &d = shapes[i];
     const int64_t tiles = ((m + d.bm - 1) / d.bm) * ((n + d.bn - 1) / d.bn);
     for (int s = 1; s <= 8 && tiles * s <= device_cus(); ++s) {
       const int64_t per = (kt + s - 1) / s;
-      if (s > 1 && (kt / s < 2 || (s - 1) * per >= kt)) continue;
-      const bool rows = mode == kDeepRowMajor && k % kTileK == 0 && per <= d.rows_max;
-      const bool relayout = mode == kDeepRowMajor && !rows;
-      if (relayout && no_relayout) continue;
+      if (s > 1 && (kt / s < min_part || (s - 1) * per >= kt)) continue;
+      const bool rows = !blocked && rows_ok && per <= d.rows_max;
+      const bool relayout = !blocked && !rows;
+      if (relayout && !relayout_ok) continue;
       const size_t parts = s > 1 ? round_up_256((size_t)s * (size_t)m * (size_t)n * sizeof(float)) : 0;
       const size_t bytes =
           parts + (relayout ? round_up_256(scale_buffer_bytes(m, k)) + round_up_256(scale_buffer_bytes(n, k)) : 0);
       if (bytes > room) continue;
       const double w = (double)(tiles * s) * scale_cus / 64.0;
       const int at = w >= 4.0 ? 3 : (int)w;
-      double us = d.fixed + (double)per * (d.step[at] + (w - at) * (d.step[at + 1] - d.step[at])) * (rows ? 1.0 + d.rows_step : 1.0);
+      double step = d.step[at] + (w - at) * (d.step[at + 1] - d.step[at]);
+      if (rows) step *= 1.0 + d.rows_step;
+      if (four_bit) step *= 0.86;
+      double us = d.fixed + (double)per * step;
       if (rows) us += d.rows;
       if (relayout) us += 4.5 + (double)(n * k) / 80.0e6;
       if (s > 1) us += d.split + 0.05 * s + 1.3e-6 * (double)s * (double)m * (double)n;
       if (us < best_us) {
         best_us = us;
-        best.shape = i, best.splits = s, best.relayout = relayout, best.bytes = bytes;
+        best.shape = d.index, best.splits = s, best.relayout = relayout, best.bytes = bytes;
       }
     }
   }
   return best;
 }
 
-hipError_t run_deep(GemmParams p, const DeepChoice &d, void *workspace, hipStream_t stream) {
+// shape < 0: not for this kernel.
+DeepChoice deep_choice(int v, int64_t m, int64_t n, int64_t k, int out_dtype, int asl, int bsl, size_t room) {
+  const DeepScaleMode mode = deep_scale_mode(k, asl, bsl);
+  bool no_relayout = false;
+  if (mode == kDeepNone || n < 1024 || k < 1024 || n % (out_dtype == WAVE_MXFP4_OUT_BF16 ? 8 : 4) != 0 ||
+      !deep_over(v, m, n, k, mode, &no_relayout))
+    return DeepChoice();
+  return deep_search(kDeepShapes, (int)(sizeof(kDeepShapes) / sizeof(kDeepShapes[0])), m, n, k, (k + kTileK - 1) / kTileK, 2,
+                     mode == kDeepBlocked, k % kTileK == 0, !no_relayout, false, room);
+}
+
+// MXFP8 operands (row-major scales; a K tile is 128 elements): every problem of one round of the deep-ring kernel's
+// tiles goes to it.  Fitted like the above to 60 random shapes (the choice at 1.004 of the best by name): 1.66 times as
+// fast as the tile kernels with their re-layout launch in the geometric mean, never behind (us: 675 x 1760 x 11136
+// 85.3 -> 35.0, 290 x 4608 x 7424 39.8 -> 23.7, 64 x 1856 x 2048 17.7 -> 8.0, 591 x 7168 x 2816 29.6 -> 25.4).
+constexpr DeepShape kDeepShapes8[] = {
+    {0, 64, 64, 31, 3.24, {0.211, 0.233, 0.228, 0.224, 0.329}, 2.0, 0.0, 1.15},
+    {2, 128, 128, 31, 3.73, {0.366, 0.371, 0.423, 0.448, 0.626}, 1.8, 0.0, 0.92},
+    {4, 256, 128, 9, 4.21, {0.568, 0.637, 0.691, 0.785, 0.912}, 1.7, 0.0, 0.93},
+};
+
+DeepChoice deep8_choice(int64_t m, int64_t n, int64_t k, int out_dtype, bool four_bit, size_t room) {
+  if (n < 1024 || k < 1024 || n % (out_dtype == WAVE_MXFP4_OUT_BF16 ? 8 : 4) != 0) return DeepChoice();
+  return deep_search(kDeepShapes8, (int)(sizeof(kDeepShapes8) / sizeof(kDeepShapes8[0])), m, n, k, k / 128, 4, false, true,
+                     k % 256 == 0, four_bit, room);
+}
+
+// a_fmt < 0: MXFP4
+hipError_t run_deep(GemmParams p, const DeepChoice &d, void *workspace, hipStream_t stream, int a_fmt = -1, int b_fmt = -1) {
   uint8_t *ws = (uint8_t *)workspace;
   hipError_t e;
   if (d.splits > 1) {
@@ -617,7 +648,7 @@ hipError_t run_deep(GemmParams p, const DeepChoice &d, void *workspace, hipStrea
     p.a_scale = ws, p.b_scale = bs;
     p.a_scale_layout = p.b_scale_layout = WAVE_MXFP4_SCALE_MFMA32;
   }
-  e = launch_deep_gemm(p, d.shape, stream);
+  e = a_fmt < 0 ? launch_deep_gemm(p, d.shape, stream) : launch_deep_gemm_fp8(p, d.shape, a_fmt, b_fmt, stream);
   if (e != hipSuccess || d.splits == 1) return e;
   return launch_splitk_reduce(p.partial, p.c, (int64_t)p.m * p.n, d.splits, p.out_bf16, stream);
 }
@@ -1044,8 +1075,13 @@ static int mxfp8_auto_split(int64_t m, int64_t n, int64_t k) {
 size_t wave_mxfp8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0 || k % 256 != 0) return 0;
   const int s = mxfp8_auto_split(m, n, k);
-  return round_up_256(scale_buffer_bytes(m, k)) + round_up_256(scale_buffer_bytes(n, k)) +
-         (s > 1 ? round_up_256((size_t)s * (size_t)m * (size_t)n * sizeof(float)) : 0);
+  size_t most = round_up_256(scale_buffer_bytes(m, k)) + round_up_256(scale_buffer_bytes(n, k)) +
+                (s > 1 ? round_up_256((size_t)s * (size_t)m * (size_t)n * sizeof(float)) : 0);
+  for (const bool four_bit : {false, true}) {
+    const size_t deep = deep8_choice(m, n, k, WAVE_MXFP4_OUT_F32, four_bit, SIZE_MAX).bytes;
+    if (deep > most) most = deep;
+  }
+  return most;
 }
 
 int wave_mxfp8_gemm(const void *a, const void *a_scale, const void *b, const void *b_scale, void *c,
@@ -1085,6 +1121,11 @@ int wave_mxfp8_gemm(const void *a, const void *a_scale, const void *b, const voi
   if (k == 0) {  // empty reduction: C = 0 (the naive kernel never touches the operands)
     p.kp = 0;
     return record_hip(launch_naive_gemm(p, stream));
+  }
+  if (variant == WAVE_MXFP4_VARIANT_AUTO) {
+    const DeepChoice d = deep8_choice(m, n, k, out_dtype, a_format == WAVE_MXFP8_B_E2M1 || b_format == WAVE_MXFP8_B_E2M1,
+                                      workspace ? workspace_bytes : 0);
+    if (d.shape >= 0) return record_hip(run_deep(p, d, workspace, stream, a_format, b_format));
   }
   int v = variant;
   if (v == WAVE_MXFP4_VARIANT_AUTO) {

@@ -150,6 +150,7 @@ bool midb_gemm_applies(const GemmParams &p);
 hipError_t launch_midb_gemm(const GemmParams &p, hipStream_t stream);
 // shape: index into kDeepShapes (mxfp4_api.hip)
 hipError_t launch_deep_gemm(const GemmParams &p, int shape, hipStream_t stream);
+hipError_t launch_deep_gemm_fp8(const GemmParams &p, int shape, int a_fmt, int b_fmt, hipStream_t stream);
 bool mid_gemm_applies(const GemmParams &p);
 hipError_t launch_mid_gemm(const GemmParams &p, int num_cus, hipStream_t stream, int bm = 0);
 bool mid_grouped_applies(const GemmParams &p);
