@@ -1344,8 +1344,8 @@ int wave_mxfp4_gemm_grouped(const void *a, const void *a_scale, const void *b, c
     const auto rm_or_native = [](int l) { return l == WAVE_MXFP4_SCALE_ROW_MAJOR || l == WAVE_MXFP4_SCALE_MFMA32; };
     if (rm_or_native(p.a_scale_layout) && rm_or_native(p.b_scale_layout) && persist_gemm_applies(q, v, device_cus())) {
       const bool a_native = p.a_scale_layout == WAVE_MXFP4_SCALE_MFMA32, b_native = p.b_scale_layout == WAVE_MXFP4_SCALE_MFMA32;
-      // (a problem of few rounds cuts a sparse last round along K instead: no short tiles then)
-      const bool cut_tail = v == WAVE_MXFP4_VARIANT_T256x256_W4x2 && grouped_tail_bytes(total_rows, n, k, num_groups) != 0;
+      // (a problem of few rounds cuts a sparse last round along K instead, in whole K tiles: no short tiles then)
+      const bool cut_tail = v == WAVE_MXFP4_VARIANT_T256x256_W4x2 && k % kTileK == 0 && grouped_tail_bytes(total_rows, n, k, num_groups) != 0;
       const int short_rows = v == WAVE_MXFP4_VARIANT_T256x256_W4x2 && !cut_tail ? kGroupedShortRows : 0;
       const GroupTableArgs gt{offsets, num_groups, 256, short_rows, (int)total_rows, table};
       if (a_native && b_native)

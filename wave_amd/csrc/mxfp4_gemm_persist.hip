@@ -600,7 +600,9 @@ __device__ __forceinline__ void persist_body(const GemmParams &p) {
   // chunk c sits at position c ^ (row % chunks per row) (conflict-free 16-byte
   // reads, two-way on the 8-byte writes), written pass by pass and read back as
   // whole rows, 16 bytes per lane.
-  // `cbase`: the tile's first row; `f32_tag`: store f32 whatever the kernel's output type (the parts of SPLIT)
+  // `cbase`: the tile's first row; `f32_tag`: store f32 whatever the kernel's output type (the parts of SPLIT).
+  // `ldc` is also where the columns end: a lane whose 16 bytes lie past the last column of C (N is a multiple of
+  // what they hold) gets an offset beyond the descriptor, so the count of stores is a whole tile's.
   auto store_tile = [&](int slot, uint8_t *cbase, int ldc, int tn0, int rows, auto f32_tag) {
     constexpr bool out_bf16 = OUT_BF16 && !decltype(f32_tag)::value;
     constexpr int SW = SLOT / NWAVES;  // staging bytes of a wave
@@ -647,11 +649,12 @@ __device__ __forceinline__ void persist_body(const GemmParams &p) {
             }
           }
           asm volatile("" ::: "memory");
+          const int past = wn0 + jg * CP + lc * 8 < ldc ? 0 : (int)0x80000000;
 #pragma unroll
           for (int r0 = 0; r0 < 32; r0 += RPI) {
             const int r = r0 + lr;
             const v4i v = *(const v4i *)(stage + r * RP + ((lc ^ (r & (NCH - 1))) << 4));
-            __builtin_amdgcn_raw_buffer_store_b128(v, c_rsrc, ((wr0 + i * 32 + r) * ldc + wn0 + jg * CP + lc * 8) * 2,
+            __builtin_amdgcn_raw_buffer_store_b128(v, c_rsrc, (((wr0 + i * 32 + r) * ldc + wn0 + jg * CP + lc * 8) * 2) | past,
                                                        0, kStorePolicy);
           }
           asm volatile("" ::: "memory");
@@ -666,11 +669,12 @@ __device__ __forceinline__ void persist_body(const GemmParams &p) {
           }
           asm volatile("" ::: "memory");
           const int lr4 = lane_v >> 2, lc4 = lane_v & 3;
+          const int past = wn0 + (MT_N - 1) * 32 + lc4 * 8 < ldc ? 0 : (int)0x80000000;
 #pragma unroll
           for (int r0 = 0; r0 < 32; r0 += 16) {
             const int r = r0 + lr4;
             const v4i v = *(const v4i *)(stage + r * RP + ((lc4 ^ (r & (NCH - 1))) << 4));
-            __builtin_amdgcn_raw_buffer_store_b128(v, c_rsrc, ((wr0 + i * 32 + r) * ldc + wn0 + (MT_N - 1) * 32 + lc4 * 8) * 2,
+            __builtin_amdgcn_raw_buffer_store_b128(v, c_rsrc, (((wr0 + i * 32 + r) * ldc + wn0 + (MT_N - 1) * 32 + lc4 * 8) * 2) | past,
                                                        0, kStorePolicy);
           }
           asm volatile("" ::: "memory");
@@ -693,12 +697,13 @@ __device__ __forceinline__ void persist_body(const GemmParams &p) {
             }
           }
           asm volatile("" ::: "memory");
+          const int past = wn0 + jg * CP + lc * 4 < ldc ? 0 : (int)0x80000000;
 #pragma unroll
           for (int r0 = 0; r0 < 32; r0 += RPI) {
             const int r = r0 + lr;
             const v4f v = *(const v4f *)(stage + r * RP + ((lc ^ (r & (NCH - 1))) << 4));
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, v), c_rsrc,
-                                                       ((wr0 + i * 32 + r) * ldc + wn0 + jg * CP + lc * 4) * 4, 0, kStorePolicy);
+                                                       (((wr0 + i * 32 + r) * ldc + wn0 + jg * CP + lc * 4) * 4) | past, 0, kStorePolicy);
           }
           asm volatile("" ::: "memory");
         }
@@ -799,7 +804,7 @@ __device__ __forceinline__ void persist_body(const GemmParams &p) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const v16f &a = acc[i][0];
-          const int off = ((i * 32 + fr) * ldc + col0 + q * 8) * ELT;
+          const int off = (((i * 32 + fr) * ldc + col0 + q * 8) * ELT) | (col0 + q * 8 < ldc ? 0 : (int)0x80000000);
           if constexpr (OUT_BF16) {
             typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
             const bf4 h = {(__bf16)a[4 * q], (__bf16)a[4 * q + 1], (__bf16)a[4 * q + 2], (__bf16)a[4 * q + 3]};
@@ -969,7 +974,7 @@ __global__ void __launch_bounds__(256) persist_tail_sum_kernel(const GemmParams 
   for (int e = threadIdx.x; e < kSumRows * BN / 4; e += 256) {
     const int row = band * kSumRows + e / (BN / 4), col = (e % (BN / 4)) * 4;
     const int m = m_first + row, n = tn * BN + col;
-    if (m >= m_end) continue;
+    if (m >= m_end || n >= p.n) continue;
     v4f sum = *(const v4f *)(part + (int64_t)row * BN + col);
     for (int i = 1; i < parts; ++i) sum += *(const v4f *)(part + ((int64_t)i * BM + row) * BN + col);
     if (p.out_bf16) {
@@ -1021,6 +1026,9 @@ template <class Cfg>
 static hipError_t launch_persist_cfg(const GemmParams &p, int grid_x, hipStream_t stream) {
   if (p.tile_table != nullptr) {
     if constexpr (Cfg::NWAVES == 8 && Cfg::BN == 256) {
+      if ((p.k & (kTileK - 1)) != 0)  // a partial last K tile (the last round is not cut then)
+        return p.out_bf16 ? launch_persist_out<Cfg, true, true, true, false>(p, grid_x, stream)
+                          : launch_persist_out<Cfg, false, true, true, false>(p, grid_x, stream);
       if (p.tail_partial != nullptr)  // few rounds: a sparsely filled last one is cut along K (decided on the device)
         return p.out_bf16 ? launch_persist_out<Cfg, true, true, false, true>(p, grid_x, stream)
                           : launch_persist_out<Cfg, false, true, false, true>(p, grid_x, stream);
@@ -1098,9 +1106,10 @@ bool persist_gemm_applies(const GemmParams &p, int variant, int num_cus) {
   const bool shuffled = p.a_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE && p.b_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE &&
                         variant != WAVE_MXFP4_VARIANT_T256x256_W2x2 && p.num_groups == 0 && (p.k & (kTileK - 1)) == 0;
   if (!shuffled && (p.a_scale_layout != WAVE_MXFP4_SCALE_MFMA32 || p.b_scale_layout != WAVE_MXFP4_SCALE_MFMA32)) return false;
-  if (p.n % bn != 0 || p.tiles_n != p.n / bn || p.k_tiles < 3) return false;  // any M
-  // a partial last K tile: dense problems with at least four K tiles
-  if ((p.k & (kTileK - 1)) != 0 && (p.num_groups != 0 || p.k_tiles < 4)) return false;
+  // any M; any N whose rows of C are whole 16-byte pieces (the gated epilogue: whole tiles, persist_gated_applies)
+  if (p.tiles_n != (p.n + bn - 1) / bn || p.k_tiles < 3) return false;
+  // a partial last K tile: at least four K tiles, grouped problems on the 8-wave 256x256 tiles
+  if ((p.k & (kTileK - 1)) != 0 && ((p.num_groups != 0 && variant != WAVE_MXFP4_VARIANT_T256x256_W4x2) || p.k_tiles < 4)) return false;
   if (p.out_bf16 ? (p.n & 7) != 0 : (p.n & 3) != 0) return false;
   // 32-bit offsets inside one operand tile, and more tiles than workgroups
   if ((int64_t)256 * p.kp >= ((int64_t)1 << 31) || (int64_t)256 * p.n * 4 >= ((int64_t)1 << 31)) return false;
@@ -1114,7 +1123,7 @@ bool persist_gemm_applies(const GemmParams &p, int variant, int num_cus) {
 bool persist_gemm_fp8_applies(const GemmParams &p, int num_cus) {
   if (p.num_groups != 0 || p.tile_table != nullptr || p.splits != 1 || p.partial != nullptr || p.b_preshuffled) return false;
   if (p.a_scale_layout != WAVE_MXFP4_SCALE_MFMA32 || p.b_scale_layout != WAVE_MXFP4_SCALE_MFMA32) return false;
-  if ((p.n & 255) != 0 || p.tiles_n != p.n / 256 || (p.k & 255) != 0 || p.k_tiles < 4) return false;
+  if ((p.n & (p.out_bf16 ? 7 : 3)) != 0 || p.tiles_n != (p.n + 255) / 256 || (p.k & 255) != 0 || p.k_tiles < 4) return false;
   if ((int64_t)256 * p.kp >= ((int64_t)1 << 31) || (int64_t)256 * p.n * 4 >= ((int64_t)1 << 31)) return false;
   const int grid = num_cus / kNumXcd * kNumXcd;
   return grid >= kNumXcd && (int64_t)p.tiles_m * p.tiles_n > grid;
@@ -1152,6 +1161,7 @@ hipError_t launch_persist_gemm_fp8(const GemmParams &p, int num_cus, int a_fmt, 
 bool persist_gated_applies(const GemmParams &p, int num_cus) {
   if (!p.out_bf16 || p.epi_scale == nullptr || (p.k & (kTileK - 1)) != 0 || p.tail_partial != nullptr || p.tail_parts > 1)
     return false;
+  if ((p.n & 255) != 0) return false;  // (whole tiles: its store has no end of the columns)
   if (p.epi_scale_layout != WAVE_MXFP4_SCALE_MFMA32) return false;
   if (p.a_scale_layout != WAVE_MXFP4_SCALE_MFMA32 || p.b_scale_layout != WAVE_MXFP4_SCALE_MFMA32) return false;
   if ((int64_t)p.m * (p.n >> 6) >= ((int64_t)1 << 31) || (int64_t)((p.m + 31) >> 5) * (((p.n >> 6) + 7) >> 3) * 256 >= ((int64_t)1 << 31))
