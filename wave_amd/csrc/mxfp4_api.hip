@@ -1251,12 +1251,12 @@ static size_t grouped_a_scale_bytes(int64_t total_rows, int64_t k) { return roun
 static size_t grouped_tail_bytes(int64_t total_rows, int64_t n, int64_t k, int num_groups) {
   const int64_t grid = device_cus() / 8 * 8;
   const int64_t tiles = (total_rows / 256 + num_groups) * (n / 256);
-  if (n % 256 != 0 || k / kTileK < 8 || grid <= 0 || tiles > 4 * grid) return 0;
+  if (n % 256 != 0 || k % kTileK != 0 || k / kTileK < 8 || grid <= 0 || tiles > 4 * grid) return 0;
   return (size_t)grid * 256 * 256 * sizeof(float);
 }
 
 size_t wave_mxfp4_grouped_workspace_bytes(int64_t total_rows, int64_t n, int64_t k, int num_groups) {
-  if (total_rows <= 0 || n <= 0 || k <= 0 || num_groups <= 0 || k % kTileK != 0 || n % 32 != 0) return 0;
+  if (total_rows <= 0 || n <= 0 || k <= 0 || num_groups <= 0 || k % 32 != 0 || n % 32 != 0) return 0;
   return grouped_table_bytes(total_rows, num_groups) + grouped_a_scale_bytes(total_rows, k) +
          round_up_256((size_t)num_groups * scale_buffer_bytes(n, k)) + grouped_tail_bytes(total_rows, n, k, num_groups);
 }
