@@ -133,7 +133,7 @@ static double table_step(const double (*tab)[2], int rows, double wgs) {
 }
 
 // us of variant `v` (128x128, 128x256 or 256x256 tiles) with `s` parts along K; negative where `s` is no valid split
-static double tile_cost_us(int v, int s, int64_t m, int64_t n, int64_t k, bool native_scales) {
+static double tile_cost_us(int v, int s, int64_t m, int64_t n, int64_t k, bool native_scales, int cus) {
   static const double t128[][2] = {{0, 0.70},    {256, 0.72},  {257, 0.82},  {320, 0.92},  {384, 0.97},
                                    {448, 1.07},  {512, 1.10},  {513, 1.58},  {640, 1.86},  {768, 1.93},
                                    {1024, 2.33}, {1025, 2.71}, {1344, 3.23}, {1792, 4.24}};
@@ -146,7 +146,7 @@ static double tile_cost_us(int v, int s, int64_t m, int64_t n, int64_t k, bool n
   const int64_t tiles = ((m + bm - 1) / bm) * ((n + bn - 1) / bn);
   const int64_t k_tiles = (k + kTileK - 1) / kTileK, per = (k_tiles + s - 1) / s;
   if (s > 1 && (k_tiles / s < 2 || (s - 1) * per >= k_tiles)) return -1.0;
-  const double wgs = (double)(tiles * s) * 256.0 / (double)device_cus();
+  const double wgs = (double)(tiles * s) * 256.0 / (double)cus;
   double fixed, step;
   if (bm == 128 && bn == 128) {
     fixed = native_scales ? 5.0 : 13.5;
@@ -159,8 +159,9 @@ static double tile_cost_us(int v, int s, int64_t m, int64_t n, int64_t k, bool n
   } else {
     fixed = native_scales ? 9.5 : 14.0;
     step = table_step(t256, sizeof(t256) / sizeof(t256[0]), wgs);
-    // (beyond one workgroup per CU the table is the persistent kernel's; an N that is not in whole 256-column tiles
-    // runs one tile per workgroup in whole rounds: 3072 x 5504 x 8192, 264 tiles, 111 us = 2 x 1.52 per K tile)
+    // (beyond one workgroup per CU the table is the persistent kernel's with its cut of a sparse last round, for which an
+    // N that is not in whole 256-column tiles gets no scratch: 3072 x 5504 x 8192, 264 tiles, 107 us against 100 on the
+    // smaller tiles that this step leads to; 3000 x 5536 x 16384 201 against 184)
     if (n % 256 != 0 && wgs > 256) step = 1.55 * (double)(((int64_t)wgs + 255) / 256);
   }
   const double reduce = s > 1 ? (native_scales ? 3.5 : 2.0) + 0.4 * s + 1.3e-6 * (double)s * (double)m * (double)n : 0.0;
@@ -188,6 +189,7 @@ static TileChoice best_tile_choice(int64_t m, int64_t n, int64_t k, bool native_
   static const int variants[] = {WAVE_MXFP4_VARIANT_T128x128_W2x2, WAVE_MXFP4_VARIANT_T128x256_W2x2,
                                  WAVE_MXFP4_VARIANT_T256x256_W4x2};
   TileChoice best = {only ? only : WAVE_MXFP4_VARIANT_T128x128_W2x2, 1, 1e30};
+  const int cus = device_cus();  // (a runtime call: once, not per candidate)
   for (int v : variants) {
     if (only && !(v == only || (v == WAVE_MXFP4_VARIANT_T256x256_W4x2 && only == WAVE_MXFP4_VARIANT_T256x256_W2x2))) continue;
     int bm, bn;
@@ -195,7 +197,7 @@ static TileChoice best_tile_choice(int64_t m, int64_t n, int64_t k, bool native_
     const int64_t tiles = ((m + bm - 1) / bm) * ((n + bn - 1) / bn);
     for (int s = 1; s <= 8; ++s) {
       if (s > 1 && tiles * s > 640) break;  // (beyond what was measured with a split, and never close)
-      const double us = tile_cost_us(v, s, m, n, k, native_scales);
+      const double us = tile_cost_us(v, s, m, n, k, native_scales, cus);
       if (us >= 0.0 && us < best.us) best = {only ? only : v, s, us};
     }
   }
@@ -571,12 +573,13 @@ bool deep_over(int v, int64_t m, int64_t n, int64_t k, DeepScaleMode mode, bool 
 DeepChoice deep_search(const DeepShape *shapes, int count, int64_t m, int64_t n, int64_t k, int64_t kt, int min_part,
                        bool blocked, bool rows_ok, bool relayout_ok, bool four_bit, size_t room) {
   DeepChoice best;
-  const double scale_cus = 256.0 / (double)device_cus();
+  const int64_t cus = device_cus();  // (a runtime call: once, not per candidate)
+  const double scale_cus = 256.0 / (double)cus;
   double best_us = 1e30;
   for (int i = 0; i < count; ++i) {
     const DeepShape &d = shapes[i];
     const int64_t tiles = ((m + d.bm - 1) / d.bm) * ((n + d.bn - 1) / d.bn);
-    for (int s = 1; s <= 8 && tiles * s <= device_cus(); ++s) {
+    for (int s = 1; s <= 8 && tiles * s <= cus; ++s) {
       const int64_t per = (kt + s - 1) / s;
       if (s > 1 && (kt / s < min_part || (s - 1) * per >= kt)) continue;
       const bool rows = !blocked && rows_ok && per <= d.rows_max;
@@ -978,7 +981,7 @@ int wave_mxfp4_gemm(const void *a, const void *a_scale, const void *b, const voi
       GemmParams p192 = p;
       p192.tiles_n = (int)(n / 192);
       if (variant == WAVE_MXFP4_VARIANT_AUTO && tv == WAVE_MXFP4_VARIANT_T256x256_W4x2 &&
-          persist_prefers_192(p, device_cus(), parts) &&
+          (persist_prefers_192(p, device_cus(), parts) || persist_192_over_tile_kernel(p, device_cus())) &&
           persist_gemm_applies(p192, WAVE_MXFP4_VARIANT_T256x192_W4x2, device_cus())) {
         // narrower tiles that fill whole rounds over the CUs
         e = launch_persist_gemm(p192, WAVE_MXFP4_VARIANT_T256x192_W4x2, device_cus(), stream);

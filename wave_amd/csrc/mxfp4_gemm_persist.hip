@@ -15,7 +15,7 @@
 // behind the loads it needs; from the second K tile on the stores must have
 // drained, which by then they have had a whole K tile of time to do.
 //
-// Taken for N % 256 == 0, K >= 768 (K % 256 != 0 with a partial last K tile from
+// Taken for any N whose rows of C are whole 16-byte pieces, K >= 768 (K % 256 != 0 with a partial last K tile from
 // K = 1024 on; any M: the last tile row reads
 // and writes through descriptors that end with the tensors), MFMA-native
 // scales for both operands, no split; grouped (MoE) problems by way of a table
@@ -1077,11 +1077,11 @@ bool persist_prefers_192(const GemmParams &p, int num_cus, int parts256) {
   return 0.785 * rounds(t192, 1) < 0.95 * rounds(t256, parts256);
 }
 
-// The same question where N is a multiple of 192 but not of 256: the 256x256 tiles then run one per workgroup, in
-// whole rounds over the CUs, and the persistent kernel on 256x192 tiles is the alternative from more tiles than
-// workgroups on, at any number of tile rows (896 x 19584 x 3584: 308 tiles in two rounds 63.3 us, 408 narrower tiles
-// 51.7; 1183 x 19584: 66.8 -> 55.4; 640 x 19584, 231 tiles in one round, stays: 38.1 against 45.4; 1536 x 19584,
-// 462 against 612 tiles, stays: 70.7 against 76.4).
+// The same question where N is a multiple of 192 but not of 256, measured against 256x256 tiles in whole rounds over the
+// CUs (which they still take on the tile kernel up to one round; the persistent kernel has no scratch to cut its last
+// round there): from more 256x192 tiles than workgroups on, at any number of tile rows (896 x 19584 x 3584: 308 tiles in
+// two rounds 63.3 us, 408 narrower tiles 51.7; 1183 x 19584: 66.8 -> 55.4; 640 x 19584, 231 tiles in one round, stays:
+// 38.1 against 45.4; 1536 x 19584, 462 against 612 tiles, stays: 70.7 against 76.4).
 bool persist_192_over_tile_kernel(const GemmParams &p, int num_cus) {
   if (p.num_groups != 0 || p.n % 192 != 0 || p.n % 256 == 0 || p.splits != 1) return false;
   const int grid = num_cus / kNumXcd * kNumXcd;
