@@ -508,20 +508,20 @@ size_t round_up_256(size_t v) { return (v + 255) / 256 * 256; }
 // ---- The deep-ring kernel (mxfp4_gemm_deep.hip): the tile shape and the parts along K for a dense problem ----
 // It runs one workgroup per CU, so it is for problems that are one round of its tiles at most.  Which shape and how many
 // parts is an estimate (us) from the same quantities as above, fitted to 300 random shapes (M = 1 .. 4096, N = 1024 ..
-// 28672, K = 1024 .. 16384, weights from HBM, every shape with 1-8 parts by name: the choice is at 1.0135 of the best
+// 28672, K = 1024 .. 16384, weights from HBM, every shape with 1-8 parts by name: the choice is at 1.010 of the best
 // of them in the geometric mean): a fixed part, a workgroup's time per K tile at 0 / 64 / 128 / 192 / 256 workgroups in
-// flight, a split's reduction, and what row-major scales cost when the workgroups stage them themselves (`rows`, up
+// flight, B's megabytes, a split's reduction, and what row-major scales cost when the workgroups stage them themselves (`rows`, up
 // to rows_max K tiles each) or when a launch in front re-lays them.
 struct DeepShape {
   int index, bm, bn, rows_max;  // index: launch_deep_gemm's shape
-  double fixed, step[5], split, rows_step, rows;
+  double fixed, step[5], split, rows_step, rows, per_mb;
 };
 constexpr DeepShape kDeepShapes[] = {
-    {0, 64, 64, 15, 3.81, {0.212, 0.246, 0.275, 0.306, 0.364}, 2.30, 0.557, 0.0},
-    {1, 64, 128, 9, 3.94, {0.308, 0.424, 0.489, 0.571, 0.674}, 2.43, 0.217, 0.2},
-    {2, 128, 128, 15, 3.63, {0.339, 0.469, 0.566, 0.613, 0.822}, 2.50, 0.365, 0.2},
-    {3, 128, 256, 5, 4.70, {0.503, 0.803, 0.926, 1.002, 1.392}, 2.04, 0.112, 0.6},
-    {4, 256, 128, 5, 5.00, {0.440, 0.618, 0.739, 0.795, 1.268}, 2.13, 0.249, 0.4},
+    {0, 64, 64, 15, 3.83, {0.209, 0.224, 0.237, 0.242, 0.298}, 2.30, 0.616, 0.0, 0.045},
+    {1, 64, 128, 9, 4.07, {0.298, 0.338, 0.357, 0.350, 0.437}, 2.39, 0.303, 0.23, 0.086},
+    {2, 128, 128, 15, 3.65, {0.337, 0.445, 0.519, 0.546, 0.743}, 2.50, 0.387, 0.17, 0.027},
+    {3, 128, 256, 5, 4.94, {0.490, 0.713, 0.776, 0.851, 1.274}, 1.85, 0.098, 0.72, 0.060},
+    {4, 256, 128, 5, 4.92, {0.448, 0.637, 0.782, 0.840, 1.340}, 2.21, 0.236, 0.40, -0.028},
 };
 struct DeepChoice {
   int shape = -1, splits = 1;
@@ -594,7 +594,7 @@ DeepChoice deep_search(const DeepShape *shapes, int count, int64_t m, int64_t n,
       double step = d.step[at] + (w - at) * (d.step[at + 1] - d.step[at]);
       if (rows) step *= 1.0 + d.rows_step;
       if (four_bit) step *= 0.86;
-      double us = d.fixed + (double)per * step;
+      double us = d.fixed + (double)per * step + d.per_mb * 1e-6 * (double)n * (double)(k / 2);
       if (rows) us += d.rows;
       if (relayout) us += 4.5 + (double)(n * k) / 80.0e6;
       if (s > 1) us += d.split + 0.05 * s + 1.3e-6 * (double)s * (double)m * (double)n;
@@ -619,13 +619,13 @@ DeepChoice deep_choice(int v, int64_t m, int64_t n, int64_t k, int out_dtype, in
 }
 
 // MXFP8 operands (row-major scales; a K tile is 128 elements): every problem of one round of the deep-ring kernel's
-// tiles goes to it.  Fitted like the above to 60 random shapes (the choice at 1.004 of the best by name): 1.66 times as
+// tiles goes to it.  Fitted like the above to 60 random shapes (the choice at 1.007 of the best by name): 1.66 times as
 // fast as the tile kernels with their re-layout launch in the geometric mean, never behind (us: 675 x 1760 x 11136
 // 85.3 -> 35.0, 290 x 4608 x 7424 39.8 -> 23.7, 64 x 1856 x 2048 17.7 -> 8.0, 591 x 7168 x 2816 29.6 -> 25.4).
 constexpr DeepShape kDeepShapes8[] = {
-    {0, 64, 64, 31, 3.24, {0.211, 0.233, 0.228, 0.224, 0.329}, 2.0, 0.0, 1.15},
-    {2, 128, 128, 31, 3.73, {0.366, 0.371, 0.423, 0.448, 0.626}, 1.8, 0.0, 0.92},
-    {4, 256, 128, 9, 4.21, {0.568, 0.637, 0.691, 0.785, 0.912}, 1.7, 0.0, 0.93},
+    {0, 64, 64, 31, 3.24, {0.211, 0.233, 0.228, 0.224, 0.329}, 2.0, 0.0, 1.15, 0.0},
+    {2, 128, 128, 31, 3.73, {0.366, 0.371, 0.423, 0.448, 0.626}, 1.8, 0.0, 0.92, 0.0},
+    {4, 256, 128, 9, 4.21, {0.568, 0.637, 0.691, 0.785, 0.912}, 1.7, 0.0, 0.93, 0.0},
 };
 
 DeepChoice deep8_choice(int64_t m, int64_t n, int64_t k, int out_dtype, bool four_bit, size_t room) {
