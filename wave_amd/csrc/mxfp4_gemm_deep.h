@@ -13,7 +13,7 @@
 //     which saves the launch that adds the parts, and the parts.
 // Measured (us per call with weights from HBM, scales resident unless said, the library's choice before -> now):
 //   1024 x 1024 x 1024 row-major scales 7.1 -> 5.6   128 x 3840 x 4096 13.5 -> 8.0    387 x 2048 x 4096 15.8 -> 8.1
-//   326 x 3584 x 5376 18.4 -> 11.9                   512 x 8192 x 8192 31.5 -> 25.2   1813 x 2624 x 9728 40.6 -> 31.6
+//   326 x 3584 x 5376 18.4 -> 11.9                   512 x 8192 x 8192 31.5 -> 23.2   1813 x 2624 x 9728 40.6 -> 31.6
 //   1000 x 7168 x 4096 24.5 -> 21.3                  2048 x 4096 x 14336 68.4 -> 59.6
 //   1 x 4096 x 6080 16.5 -> 8.6                      727 x 4096 x 11008 row-major 43.4 -> 34.1
 // MXFP8 (the tile kernels with their re-layout launch before -> now): 675 x 1760 x 11136 85.3 -> 35.0, 290 x 4608 x 7424
