@@ -85,7 +85,9 @@ template <class Cfg, int SC, int FMT, int FMT_B>
 __device__ __forceinline__ void deep_body(const GemmParams &p) {
   constexpr bool FP8 = FMT != 4 || FMT_B != 4, A4 = FP8 && FMT == 4, B4 = FP8 && FMT_B == 4;
   constexpr int STEPS = FP8 ? 2 : 4, kUnit = FP8 ? 4 : 8;
-  typedef typename std::conditional<FP8, uint32_t, uint2>::type RowUnit;
+  // (64 bits as one scalar: in front of a read of HIP's uint2 from LDS the compiler waits for every outstanding request,
+  // and where a branch loads a vector it copies it, and so waits, before the next load; see the staging below)
+  typedef typename std::conditional<FP8, uint32_t, uint64_t>::type RowUnit;
   static_assert(!FP8 || SC != kDeepShuffled, "MXFP8 scales: MFMA32 order or row-major");
   constexpr int BM = Cfg::BM, BN = Cfg::BN, MT_M = Cfg::MT_M, MT_N = Cfg::MT_N, S = Cfg::STAGES;
   constexpr int NWAVES = Cfg::NWAVES, A_LD = Cfg::A_LD, B_LD = Cfg::B_LD, S_LD = SC == kDeepRows ? 0 : Cfg::S_LD;
@@ -201,7 +203,7 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
     if constexpr (SC == kDeepRows) {
       const RowUnit v = *(const RowUnit *)(rows + (uint32_t)(blk * 32 + fr) * pitch + j * kUnit);
       if constexpr (FP8) return __builtin_amdgcn_perm(0u, v, fg ? 0x0c0c0301u : 0x0c0c0200u);
-      else return __builtin_amdgcn_perm(v.y, v.x, pick);
+      else return __builtin_amdgcn_perm((uint32_t)(v >> 32), (uint32_t)v, pick);
     } else if constexpr (SC == kDeepShuffled) {
       const uint8_t *b = s_ring + slot * Cfg::S_STAGE + blk * 256 + fg * 64 + (fr & 15) * 4;
       return __builtin_amdgcn_perm(*(const uint32_t *)(b + 128), *(const uint32_t *)b,
@@ -244,9 +246,11 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
   typedef std::integral_constant<int, 0> T0;
   typedef std::integral_constant<int, 1> T1;
   typedef std::integral_constant<int, 2> T2;
-  // inside a phase: one MFMA, the next step's fragment reads, then MFMAs and requests in turn
-  auto order_phase = [&]() {
-    constexpr int Q = MT_M * MT_N, NQ = (REQ + STEPS - 1) / STEPS;
+  typedef std::integral_constant<int, 3> T3;
+  // inside a phase: one MFMA, the next step's fragment reads, then MFMAs and the requests of share PH in turn
+  auto order_phase = [&](auto ph_tag) {
+    constexpr int PH = decltype(ph_tag)::value;
+    constexpr int Q = MT_M * MT_N, NQ = REQ * (PH + 1) / STEPS - REQ * PH / STEPS;
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
     __builtin_amdgcn_sched_group_barrier(0x100, MT_M * (int)(sizeof(FragA) / 16) + MT_N * (int)(sizeof(FragB) / 16), 0);
 #pragma unroll
@@ -265,13 +269,27 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
   FragB fb0[MT_N], fb1[MT_N];
   constexpr int kIters = SC == kDeepRows ? ((BM > BN ? BM : BN) * rows_max_k_tiles<Cfg>(kUnit) + Cfg::NT - 1) / Cfg::NT : 1;
   RowUnit row_a[kIters], row_b[kIters];
+  // unit `it` of this thread: K tile c of row r (the quotient is exact up to u * (nkt - 1) = 2^18)
+  static_assert(kIters * Cfg::NT * (kUnit == 8 ? 14 : 30) < 1 << 18, "units of the staged rows");
+  const int per_row = SC == kDeepRows ? ((1 << 18) + nkt - 1) / nkt : 0;
+  auto row_unit = [&](int it, int &r, int &c) {
+    const int u = it * Cfg::NT + (int)threadIdx.x;
+    r = (u * per_row) >> 18;
+    c = u - r * nkt;
+  };
   if constexpr (SC == kDeepRows) {
+    // All loads are in flight together, and stay so: the first round is not behind a branch and nothing is zeroed in front,
+    // or the compiler joins the branches with copies and waits for each load before the next.  With that and without a
+    // drain of the ring per K tile (the uint2 above): 1024 x 1024 x 3840, scales row-major, 10.0 -> 8.2 us, 1024 x 3840
+    // x 3840 17.1 -> 14.0, 512 x 2048 x 2048 8.3 -> 7.3, 1000 x 7168 x 1280 13.2 -> 12.0.
 #pragma unroll
-    for (int it = 0; it < kIters; ++it) {  // unit u: K tile u % nkt of row u / nkt
-      const int u = it * Cfg::NT + (int)threadIdx.x, r = u / nkt, c = u - r * nkt;
-      row_a[it] = row_b[it] = RowUnit{};
-      if (r < BM) row_a[it] = *(const RowUnit *)(p.a_scale + (int64_t)min(m0 + r, p.m - 1) * p.ks + (kt_begin + c) * kUnit);
-      if (r < BN) row_b[it] = *(const RowUnit *)(p.b_scale + (int64_t)min(n0 + r, p.n - 1) * p.ks + (kt_begin + c) * kUnit);
+    for (int it = 0; it < kIters; ++it) {
+      int r, c;
+      row_unit(it, r, c);
+      if (it == 0 || r < BM)
+        row_a[it] = *(const RowUnit *)(p.a_scale + (int64_t)min(m0 + min(r, BM - 1), p.m - 1) * p.ks + (kt_begin + c) * kUnit);
+      if (it == 0 || r < BN)
+        row_b[it] = *(const RowUnit *)(p.b_scale + (int64_t)min(n0 + min(r, BN - 1), p.n - 1) * p.ks + (kt_begin + c) * kUnit);
     }
   }
 #pragma unroll
@@ -280,7 +298,8 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
   if constexpr (SC == kDeepRows) {
 #pragma unroll
     for (int it = 0; it < kIters; ++it) {
-      const int u = it * Cfg::NT + (int)threadIdx.x, r = u / nkt, c = u - r * nkt;
+      int r, c;
+      row_unit(it, r, c);
       if (r < BM) *(RowUnit *)(rows + (uint32_t)r * pitch + c * kUnit) = row_a[it];
       if (r < BN) *(RowUnit *)(rows + (uint32_t)(BM + r) * pitch + c * kUnit) = row_b[it];
     }
@@ -301,18 +320,18 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
     read_frags(slot, 1, fa1, fb1);
     mfma_block(fa0, fb0, T0{});
     if (NEXT) issue(jr, slot_prev, WAVE_Q(1), WAVE_Q(2));
-    order_phase();
+    order_phase(T1{});
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (!FP8) {
       read_frags(slot, 2, fa0, fb0);
       mfma_block(fa1, fb1, T1{});
       if (NEXT) issue(jr, slot_prev, WAVE_Q(2), WAVE_Q(3));
-      order_phase();
+      order_phase(T2{});
       __builtin_amdgcn_sched_barrier(0);
       read_frags(slot, 3, fa1, fb1);
       mfma_block(fa0, fb0, T2{});
       if (NEXT) issue(jr, slot_prev, WAVE_Q(3), WAVE_Q(4));
-      order_phase();
+      order_phase(T3{});
       __builtin_amdgcn_sched_barrier(0);
     }
     if (NEXT) {
@@ -326,7 +345,7 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
     }
     mfma_block(fa1, fb1, std::integral_constant<int, STEPS - 1>{});
     if (NEXT) issue(j + S, slot, WAVE_Q(0), WAVE_Q(1));
-    order_phase();
+    order_phase(T0{});
     __builtin_amdgcn_sched_barrier(0);
     if (NEXT) {
 #pragma unroll
