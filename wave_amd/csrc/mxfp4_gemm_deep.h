@@ -5,7 +5,11 @@
 // the tile kernel (mxfp4_gemm_tile.hip), which is sized for two workgroups per CU and for the matrix pipes, gives the
 // second half of a K tile of B a lead of three quarters of a K tile, and its per-lane scale loads, one K tile ahead in
 // the same in-order queue, no more: 0.72 us per K tile of a 128x128 tile, whose MFMAs take 0.2.  Here
-//   * all 160 KB of LDS are one ring of 3 (128x256, 256x128) to 8 (64x64) whole K tiles, requested that many ahead;
+//   * LDS is one ring of 3 (128x256, 256x128) or 4 whole K tiles (a stream of B with few rows: 8 of 64x64), requested that
+//     many ahead.  More of the small tiles than four only put requests in front of the first K tile, which the workgroup
+//     issues before it can wait for it (64x64 with 8 -> 4, 64x128 with 6 -> 4; us by name: 1024 x 1024 x 1024 5.1 -> 4.6,
+//     1024 x 1024 x 3840 8.3 -> 7.6, 512 x 2048 x 2048 7.2 -> 6.6, 64 x 14336 x 4096 12.7 -> 11.9; over 3000 random calls the
+//     ones on these tiles take 0.94 of the time);
 //   * the scales travel in the ring too (one 256-byte block per 32 rows and K tile, four bytes per lane), so that no
 //     load that returns to a register stands in the queue in front of the operands; row-major scales of a short K
 //     range are staged once per workgroup instead, and then no launch has to re-lay them;
@@ -21,8 +25,8 @@
 //   40.2 -> 23.4, 64 x 1856 x 2048 18.7 -> 7.7, 907 x 1024 x 2560 20.3 -> 9.4.
 // Eight waves (two per SIMD) beat four on 128x128 by 1-4 % and on 128x256 by 3-9 %; 64x256 tiles and more than one round
 // (two workgroups of the tile kernel share a CU there, and the persistent kernel streams across tiles) lost and are not
-// built.  A time per K tile of 0.23-0.34 us at 64x64 up to 1.05 at 128x256 leaves the fixed part (launch, first K tile,
-// C: 3.8-5.7 us) as what bounds short K.  On a full grid of the largest tiles it is the step: 2048 x 4096 x 14336 takes 65 us on
+// built.  A time per K tile of 0.22-0.31 us at 64x64 up to 1.05 at 128x256 leaves the fixed part (launch, first K tile,
+// C: 3.5-5.7 us) as what bounds short K.  On a full grid of the largest tiles it is the step: 2048 x 4096 x 14336 takes 65 us on
 // random operands and 51 on zeros (256x128: 63 and 51), so a fifth is the matrix pipes' power limit; what holds the rest
 // back is not established.
 #ifndef WAVE_MXFP4_GEMM_DEEP_H_
@@ -59,8 +63,8 @@ struct DeepCfg {
 template <class R, class F>
 R with_deep_shape(int shape, R none, F f) {
   switch (shape) {
-    case 0: return f(DeepCfg<64, 64, 2, 2, 8>{});
-    case 1: return f(DeepCfg<64, 128, 2, 2, 6>{});
+    case 0: return f(DeepCfg<64, 64, 2, 2, 4>{});
+    case 1: return f(DeepCfg<64, 128, 2, 2, 4>{});
     case 2: return f(DeepCfg<128, 128, 2, 4, 4>{});
     case 3: return f(DeepCfg<128, 256, 2, 4, 3>{});
     case 4: return f(DeepCfg<256, 128, 4, 2, 3>{});
