@@ -250,7 +250,8 @@ size_t wave_mxfp8_workspace_bytes(int64_t m, int64_t n, int64_t k);
  * named by the caller, for tests and for measuring the library's own choice of
  * them: operands as wave_mxfp4_gemm (both formats WAVE_MXFP8_E2M1) or
  * wave_mxfp8_gemm, both scale tensors in scale_layout.  shape: 0 = 64x64,
- * 1 = 64x128, 2 = 128x128, 3 = 128x256, 4 = 256x128 (MXFP8: 0, 2 and 4); parts:
+ * 1 = 64x128, 2 = 128x128, 3 = 128x256, 4 = 256x128, 8 = 128x192 (MXFP8: 0, 2
+ * and 4); parts:
  * 1 .. 8, none of them empty; relayout = 1: row-major scales are re-laid by a
  * launch in front instead of staged by the workgroups, which take 5 to 15 K
  * tiles a part (MXFP8: 9 to 31 of 128 elements).  workspace: 4 * parts * M * N

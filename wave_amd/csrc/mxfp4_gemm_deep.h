@@ -5,14 +5,15 @@
 // the tile kernel (mxfp4_gemm_tile.hip), which is sized for two workgroups per CU and for the matrix pipes, gives the
 // second half of a K tile of B a lead of three quarters of a K tile, and its per-lane scale loads, one K tile ahead in
 // the same in-order queue, no more: 0.72 us per K tile of a 128x128 tile, whose MFMAs take 0.2.  Here
-//   * LDS is one ring of 3 (128x256, 256x128) or 4 whole K tiles (a stream of B with few rows: 8 of 64x64), requested that
+//   * LDS is one ring of 3 (128x256, 256x128, 128x192) or 4 whole K tiles (a stream of B with few rows: 8 of 64x64), requested that
 //     many ahead.  More of the small tiles than four only put requests in front of the first K tile, which the workgroup
 //     issues before it can wait for it (64x64 with 8 -> 4, 64x128 with 6 -> 4; us by name: 1024 x 1024 x 1024 5.1 -> 4.6,
 //     1024 x 1024 x 3840 8.3 -> 7.6, 512 x 2048 x 2048 7.2 -> 6.6, 64 x 14336 x 4096 12.7 -> 11.9; over 3000 random calls the
 //     ones on these tiles take 0.94 of the time);
 //   * the scales travel in the ring too (one 256-byte block per 32 rows and K tile, four bytes per lane), so that no
-//     load that returns to a register stands in the queue in front of the operands; row-major scales of a short K
-//     range are staged once per workgroup instead, and then no launch has to re-lay them;
+//     load that returns to a register stands in the queue in front of the operands; row-major scales of up to 31 K tiles
+//     (the largest tiles: 5, 128x192: 11) are staged once per workgroup instead, and then no launch has to re-lay them
+//     (186 x 4832 x 5888 17.0 -> 10.9 us, 644 x 5888 x 2304 17.1 -> 12.0);
 //   * the tiles are small enough for the problem to reach most CUs without a split along K (64x64 up to 256 of them),
 //     which saves the launch that adds the parts, and the parts.
 // Measured (us per call through the C ABI, weights from HBM, bf16 C, scales resident unless said, the kernel that the library
@@ -23,6 +24,9 @@
 //   727 x 4096 x 11008 row-major 43.0 -> 34.1
 // MXFP8 (the tile kernels with their re-layout launch before -> now): 675 x 1760 x 11136 111 -> 37, 290 x 4608 x 7424
 //   40.2 -> 23.4, 64 x 1856 x 2048 18.7 -> 7.7, 907 x 1024 x 2560 20.3 -> 9.4.
+// 128x192 tiles lie between: 526 x 7424 x 3584 15.6 (on 256x128) -> 14.2, 256 x 24576 x 8192 37.9 -> 35.4; among random shapes that
+// take them 0.93 of the time.  Tiles of an odd count of 32 columns (64x96 .. 128x224, the waves in two halves of K whose
+// sums meet in LDS) were no faster than the even ones beside them, and are not built.
 // Eight waves (two per SIMD) beat four on 128x128 by 1-4 % and on 128x256 by 3-9 %; 64x256 tiles and more than one round
 // (two workgroups of the tile kernel share a CU there, and the persistent kernel streams across tiles) lost and are not
 // built.  A time per K tile of 0.22-0.31 us at 64x64 up to 1.05 at 128x256 leaves the fixed part (launch, first K tile,
@@ -68,6 +72,7 @@ R with_deep_shape(int shape, R none, F f) {
     case 2: return f(DeepCfg<128, 128, 2, 4, 4>{});
     case 3: return f(DeepCfg<128, 256, 2, 4, 3>{});
     case 4: return f(DeepCfg<256, 128, 4, 2, 3>{});
+    case 8: return f(DeepCfg<128, 192, 4, 2, 3>{});
     default: return none;
   }
 }
@@ -76,8 +81,7 @@ R with_deep_shape(int shape, R none, F f) {
 template <class Cfg>
 __host__ __device__ constexpr int rows_max_k_tiles(int unit) {
   const int units = (160 * 1024 - Cfg::RING) / ((Cfg::BM + Cfg::BN) * unit), odd = units - 1 + units % 2;
-  const int most = unit == 8 ? 15 : 31;
-  return odd < most ? odd : most;
+  return odd < 31 ? odd : 31;
 }
 
 __host__ __device__ constexpr int rows_pitch(int nkt, int unit) { return (nkt + 1 - (nkt & 1)) * unit; }
@@ -274,8 +278,9 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
   constexpr int kIters = SC == kDeepRows ? ((BM > BN ? BM : BN) * rows_max_k_tiles<Cfg>(kUnit) + Cfg::NT - 1) / Cfg::NT : 1;
   RowUnit row_a[kIters], row_b[kIters];
   // unit `it` of this thread: K tile c of row r (the quotient is exact up to u * (nkt - 1) = 2^18)
-  static_assert(kIters * Cfg::NT * (kUnit == 8 ? 14 : 30) < 1 << 18, "units of the staged rows");
+  static_assert(kIters * Cfg::NT * 30 < 1 << 18, "units of the staged rows");
   const int per_row = SC == kDeepRows ? ((1 << 18) + nkt - 1) / nkt : 0;
+  const int units = (BM > BN ? BM : BN) * nkt;
   auto row_unit = [&](int it, int &r, int &c) {
     const int u = it * Cfg::NT + (int)threadIdx.x;
     r = (u * per_row) >> 18;
@@ -286,8 +291,10 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
     // or the compiler joins the branches with copies and waits for each load before the next.  With that and without a
     // drain of the ring per K tile (the uint2 above): 1024 x 1024 x 3840, scales row-major, 10.0 -> 8.2 us, 1024 x 3840
     // x 3840 17.1 -> 14.0, 512 x 2048 x 2048 8.3 -> 7.3, 1000 x 7168 x 1280 13.2 -> 12.0.
+    // (Rounds that the range does not need are left out whole: 1024 x 1024 x 1024 5.0 -> 4.75, 512 x 2048 x 2048 7.8 -> 7.15.)
 #pragma unroll
     for (int it = 0; it < kIters; ++it) {
+      if (it > 0 && it * Cfg::NT >= units) continue;
       int r, c;
       row_unit(it, r, c);
       if (it == 0 || r < BM)
@@ -302,6 +309,7 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
   if constexpr (SC == kDeepRows) {
 #pragma unroll
     for (int it = 0; it < kIters; ++it) {
+      if (it > 0 && it * Cfg::NT >= units) continue;
       int r, c;
       row_unit(it, r, c);
       if (r < BM) *(RowUnit *)(rows + (uint32_t)r * pitch + c * kUnit) = row_a[it];
@@ -375,7 +383,7 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
   const int64_t ldc = p.n;
   const int wm0 = m0 + wave_m * Cfg::WM, wn0 = n0 + wave_n * Cfg::WN;
   if (!to_partial && p.out_bf16) {
-    constexpr int ROWB = Cfg::WN * 2 + 8, LPR = Cfg::WN * 2 / 16, RPI = 64 / LPR;
+    constexpr int ROWB = Cfg::WN * 2 + 8, LPR = Cfg::WN * 2 / 16;
     typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
     uint8_t *stage = smem + wave * (Cfg::WM * (Cfg::WN * 4 + 16));
 #pragma unroll
@@ -390,15 +398,14 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
         }
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));
-    const int lr = lane / LPR, lc = lane % LPR;
 #pragma unroll
-    for (int r0 = 0; r0 < Cfg::WM; r0 += RPI) {
-      const int r = r0 + lr, m = wm0 + r, n = wn0 + lc * 8;
+    for (int u0 = 0; u0 < Cfg::WM * LPR; u0 += 64) {  // (64 pieces of 16 bytes at a time, WM being whole 32 rows)
+      const int r = (u0 + lane) / LPR, lc = u0 + lane - r * LPR, m = wm0 + r, n = wn0 + lc * 8;
       const v4i v = *(const v4i *)(stage + r * ROWB + lc * 16);
       if (m < p.m && n < p.n) *(v4i *)((__bf16 *)p.c + (int64_t)m * ldc + n) = v;
     }
   } else {
-    constexpr int ROWB = Cfg::WN * 4 + 16, LPR = Cfg::WN * 4 / 16, RPI = 64 / LPR;
+    constexpr int ROWB = Cfg::WN * 4 + 16, LPR = Cfg::WN * 4 / 16;
     uint8_t *stage = smem + wave * (Cfg::WM * ROWB);
 #pragma unroll
     for (int i = 0; i < MT_M; ++i)
@@ -412,10 +419,9 @@ __device__ __forceinline__ void deep_body(const GemmParams &p) {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));
     float *cbase = to_partial ? p.partial + (int64_t)split * p.m * ldc : (float *)p.c;
-    const int lr = lane / LPR, lc = lane % LPR;
 #pragma unroll
-    for (int r0 = 0; r0 < Cfg::WM; r0 += RPI) {
-      const int r = r0 + lr, m = wm0 + r, n = wn0 + lc * 4;
+    for (int u0 = 0; u0 < Cfg::WM * LPR; u0 += 64) {
+      const int r = (u0 + lane) / LPR, lc = u0 + lane - r * LPR, m = wm0 + r, n = wn0 + lc * 4;
       const v4f v = *(const v4f *)(stage + r * ROWB + lc * 16);
       if (m < p.m && n < p.n) *(v4f *)(cbase + (int64_t)m * ldc + n) = v;
     }

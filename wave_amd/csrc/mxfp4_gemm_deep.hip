@@ -10,17 +10,22 @@ namespace {
 // that of four, mean: up to 16 rows 0.96 preshuffled and 1.00 row-major, 17 .. 32 preshuffled 0.95, more rows 1.02 - 1.04).
 typedef DeepCfg<64, 64, 2, 2, 8> DeepStream;
 
+// Staged row-major scales of 128x128 tiles: a ring of three K tiles leaves room for 31 of them instead of 15 (1792 x 2048 x
+// 2304 9.4 us with either).
+template <class Cfg>
+using DeepRowsCfg = typename std::conditional<Cfg::BM == 128 && Cfg::BN == 128, DeepCfg<128, 128, 2, 4, 3>, Cfg>::type;
+
 template <class Cfg>
 hipError_t launch_deep_scales(const GemmParams &p, hipStream_t stream) {
-  if constexpr (Cfg::BM == 64 && Cfg::BN == 64 && Cfg::STAGES != DeepStream::STAGES)
-    if (p.m <= (p.b_preshuffled ? 32 : 16) && p.tiles_per_split > 16 && p.a_scale_layout != WAVE_MXFP4_SCALE_ROW_MAJOR)
-      return launch_deep_scales<DeepStream>(p, stream);
-  if (p.a_scale_layout == WAVE_MXFP4_SCALE_MFMA32 && p.b_scale_layout == WAVE_MXFP4_SCALE_MFMA32)
-    return launch_deep_cfg<Cfg, kDeepNative>(p, stream);
-  if (p.a_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE && p.b_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE)
-    return launch_deep_cfg<Cfg, kDeepShuffled>(p, stream);
-  if (p.tiles_per_split > rows_max_k_tiles<Cfg>(8)) return hipErrorInvalidValue;
-  return launch_deep_cfg<Cfg, kDeepRows>(p, stream);
+  const bool native = p.a_scale_layout == WAVE_MXFP4_SCALE_MFMA32 && p.b_scale_layout == WAVE_MXFP4_SCALE_MFMA32;
+  const bool shuffled = p.a_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE && p.b_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE;
+  if constexpr (Cfg::BM == 64 && Cfg::BN == 64)
+    if ((native || shuffled) && p.m <= (p.b_preshuffled ? 32 : 16) && p.tiles_per_split > 16)
+      return native ? launch_deep_cfg<DeepStream, kDeepNative>(p, stream) : launch_deep_cfg<DeepStream, kDeepShuffled>(p, stream);
+  if (native) return launch_deep_cfg<Cfg, kDeepNative>(p, stream);
+  if (shuffled) return launch_deep_cfg<Cfg, kDeepShuffled>(p, stream);
+  if (p.tiles_per_split > rows_max_k_tiles<DeepRowsCfg<Cfg>>(8)) return hipErrorInvalidValue;
+  return launch_deep_cfg<DeepRowsCfg<Cfg>, kDeepRows>(p, stream);
 }
 
 }  // namespace
@@ -30,7 +35,7 @@ hipError_t launch_deep_gemm(const GemmParams &p, int shape, hipStream_t stream) 
 }
 
 int deep_rows_max(int shape, bool fp8) {
-  return with_deep_shape(shape, 0, [&](auto cfg) { return rows_max_k_tiles<decltype(cfg)>(fp8 ? 4 : 8); });
+  return with_deep_shape(shape, 0, [&](auto cfg) { return fp8 ? rows_max_k_tiles<decltype(cfg)>(4) : rows_max_k_tiles<DeepRowsCfg<decltype(cfg)>>(8); });
 }
 
 }  // namespace wave_mxfp4
