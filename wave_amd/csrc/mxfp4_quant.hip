@@ -40,12 +40,11 @@ struct Elems {
   static constexpr int kDwords = 2 * kBytes;
   uint32_t d[kDwords];
 
-  __device__ __forceinline__ void load(const uint8_t *p, bool ok) {
+  template <bool ONCE>
+  __device__ __forceinline__ void load(const uint8_t *p) {
 #pragma unroll
     for (int i = 0; i < kDwords / 4; ++i) {
-      v4i v = {0, 0, 0, 0};
-      // read once: 16-bit inputs bypass the caches; an f32 lane's two loads share lines and are faster through them
-      if (ok) v = kBytes == 2 ? __builtin_nontemporal_load((const v4i *)(p + 16 * i)) : *(const v4i *)(p + 16 * i);
+      const v4i v = ONCE ? __builtin_nontemporal_load((const v4i *)(p + 16 * i)) : *(const v4i *)(p + 16 * i);
       d[4 * i + 0] = v.x, d[4 * i + 1] = v.y, d[4 * i + 2] = v.z, d[4 * i + 3] = v.w;
     }
   }
@@ -104,6 +103,7 @@ struct QuantParams {
   int src_rows;            // rows of x (a row id at or beyond src_rows * row_div yields a zero row)
   int row_div;
   int scale_layout;
+  bool stream_q;           // whether q is stored non-temporal
 };
 
 // silu(g) * u in f32, rounded to the 16-bit storage type (the value the unfused
@@ -137,8 +137,12 @@ __device__ __forceinline__ uint32_t gated_pair(uint32_t g2, uint32_t u2) {
 // takes 8 of the rows.  Four lanes share a scale group (8 elements each); the 16
 // quads of a wave take 16 consecutive groups of a row per pass, so that one load
 // instruction covers up to 1 KB (bf16) and one store 256 B of a row.
-// GATED: the elements are silu(x) * up of two 16-bit operands.
-template <int DT, int TC, bool GATED>
+// GATED: the elements are silu(x) * up of two 16-bit operands.  GATHER: rows by p.row_ids.  LAYOUT: of the scales.
+// Every lane loads: one beyond the last row, the last group or the ids loads the nearest there is and its data are zeroed
+// (a load behind a branch is waited for before the next one is issued), and the layout and the gather are compiled in.  With
+// both at run time a pass had ten branches, and a launch of few rows is bound by such latencies: 1000 x 4096 bf16 4.45 -> 3.9
+// us, 128 gathered rows of 8192 5.2 -> 3.9; a linear call (quantiser and GEMM, GPU time) of 111 x 6464 x 2304 9.8 -> 8.7.
+template <int DT, int TC, bool GATED, bool GATHER, int LAYOUT, bool ONCE>
 __global__ void __launch_bounds__(256) quantize_kernel(const QuantParams p) {
   constexpr int kEb = Elems<DT>::kBytes;
   constexpr int kGroups = 8 * TC;              // scale groups of a tile row
@@ -150,9 +154,9 @@ __global__ void __launch_bounds__(256) quantize_kernel(const QuantParams p) {
   __shared__ uint32_t tile_scales[kQuantRows * kGroups / 4];
   uint8_t *tile_bytes = (uint8_t *)tile_scales;
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int quad = lane >> 2, sub = lane & 3;
-  const int rows = p.rows, k = p.k, scale_layout = p.scale_layout;
+  const int rows = p.rows, k = p.k;
   const int ks = k >> 5, ksp = (ks + 7) & ~7;
   const int col_tiles = (ks + kGroups - 1) / kGroups;
   const int row_tile = blockIdx.x / col_tiles, col_tile = blockIdx.x - row_tile * col_tiles;
@@ -161,44 +165,52 @@ __global__ void __launch_bounds__(256) quantize_kernel(const QuantParams p) {
   // gathered rows: the ids of the wave's 8 rows, one per lane, fetched once (a load per unit would put two
   // dependent memory round trips in front of every batch)
   // ... and divided once: wave_src is the source row, or one past the last for "no such row"
-  uint32_t wave_src = (uint32_t)p.src_rows;
-  if (p.row_ids != nullptr && lane < 8 && row0 + wave * 8 + lane < rows)
-    wave_src = min((uint32_t)p.row_ids[row0 + wave * 8 + lane] / (uint32_t)p.row_div, (uint32_t)p.src_rows);
+  uint32_t wave_src = 0;
+  if constexpr (GATHER) {
+    const int r = row0 + wave * 8 + (lane & 7);
+    wave_src = min((uint32_t)p.row_ids[min(r, rows - 1)] / (uint32_t)p.row_div, (uint32_t)p.src_rows);
+  }
 
   for (int pb = 0; pb < kPasses; pb += kB) {
     Elems<DT> e[kB], eu[GATED ? kB : 1];
-    int lrow[kB], lgrp[kB];
+    bool ok[kB];
 #pragma unroll
     for (int i = 0; i < kB; ++i) {
       const int u = (pb + i) * 16 + quad;  // unit of the wave: (row, group)
-      lrow[i] = wave * 8 + u / kGroups;
-      lgrp[i] = u % kGroups;
-      const int row = row0 + lrow[i], g = g0 + lgrp[i];
-      bool ok = row < rows && g < ks;
-      int64_t src = row;
-      if (p.row_ids) {  // gathered rows
-        src = (uint32_t)__shfl((int)wave_src, u / kGroups, 64);
-        ok = ok && src < p.src_rows;
+      const int row = row0 + wave * 8 + u / kGroups, g = g0 + u % kGroups;
+      ok[i] = row < rows && g < ks;
+      int64_t src = min(row, rows - 1);
+      if constexpr (GATHER) {
+        const int id = __shfl((int)wave_src, u / kGroups, 64);
+        ok[i] = ok[i] && id < p.src_rows;
+        src = min(id, p.src_rows - 1);
       }
-      const int64_t col = (int64_t)g * 32 + sub * 8;
-      e[i].load(p.x + (src * p.ld_x + col) * kEb, ok);
-      if constexpr (GATED) eu[i].load(p.up + (src * p.ld_up + col) * kEb, ok);
+      const int64_t col = (int64_t)min(g, ks - 1) * 32 + sub * 8;
+      e[i].template load<ONCE>(p.x + (src * p.ld_x + col) * kEb);
+      if constexpr (GATED) eu[i].template load<ONCE>(p.up + (src * p.ld_up + col) * kEb);
     }
 #pragma unroll
     for (int i = 0; i < kB; ++i) {
-      const int row = row0 + lrow[i], g = g0 + lgrp[i];
+      const int u = (pb + i) * 16 + quad, lrow = wave * 8 + u / kGroups, lgrp = u % kGroups;
+      const int row = row0 + lrow, g = g0 + lgrp;
       if constexpr (GATED) {
 #pragma unroll
         for (int w = 0; w < Elems<DT>::kDwords; ++w) e[i].d[w] = gated_pair<DT>(e[i].d[w], eu[i].d[w]);
       }
+#pragma unroll
+      for (int w = 0; w < Elems<DT>::kDwords; ++w) e[i].d[w] = ok[i] ? e[i].d[w] : 0u;
       const uint32_t sb = scale_byte_of(quad_max(e[i].amax_bits()));
       const float sf = __builtin_bit_cast(float, sb ? sb << 23 : 0x00400000u);  // 2^(sb-127)
       const uint32_t codes = e[i].convert(sf);
-      if (row < rows && g < ks) __builtin_nontemporal_store(codes, (uint32_t *)(p.q + (int64_t)row * (k >> 1) + g * 16 + sub * 4));
+      if (row < rows && g < ks) {
+        uint32_t *q = (uint32_t *)(p.q + (int64_t)row * (k >> 1) + g * 16 + sub * 4);
+        if (p.stream_q) __builtin_nontemporal_store(codes, q);
+        else *q = codes;
+      }
       if (sub == 0) {
-        const int at = scale_layout == WAVE_MXFP4_SCALE_ROW_MAJOR
-                           ? lrow[i] * kGroups + lgrp[i]
-                           : (lgrp[i] >> 3) * 256 + (int)scale_offset(scale_layout, lrow[i], lgrp[i] & 7, 8, 8);
+        const int at = LAYOUT == WAVE_MXFP4_SCALE_ROW_MAJOR
+                           ? lrow * kGroups + lgrp
+                           : (lgrp >> 3) * 256 + (int)scale_offset(LAYOUT, lrow, lgrp & 7, 8, 8);
         tile_bytes[at] = (uint8_t)sb;
       }
     }
@@ -206,7 +218,7 @@ __global__ void __launch_bounds__(256) quantize_kernel(const QuantParams p) {
   __syncthreads();
 
   uint8_t *scale = p.scale;
-  if (scale_layout == WAVE_MXFP4_SCALE_ROW_MAJOR) {
+  if constexpr (LAYOUT == WAVE_MXFP4_SCALE_ROW_MAJOR) {
     // kGroups bytes of each row are contiguous
     if ((ks & 3) == 0) {
       for (int d = threadIdx.x; d < kQuantRows * kGroups / 4; d += 256) {
@@ -224,14 +236,43 @@ __global__ void __launch_bounds__(256) quantize_kernel(const QuantParams p) {
     // the tile's TC blocks of 256 bytes follow one another (padding rows and groups hold 0)
     const int k_tiles = ksp >> 3;
     uint32_t *out = (uint32_t *)(scale + ((int64_t)row_tile * k_tiles + (int64_t)col_tile * TC) * 256);
-    for (int d = threadIdx.x; d < TC * 64; d += 256) {
-      if (col_tile * TC + (d >> 6) < k_tiles) out[d] = tile_scales[d];
-    }
+    const int d = threadIdx.x;
+    static_assert(TC * 64 <= 256, "a thread per dword of the tile's scales");
+    if (d < TC * 64 && col_tile * TC + (d >> 6) < k_tiles) out[d] = tile_scales[d];
   }
 }
 
+__global__ void __launch_bounds__(256) zero_bytes_kernel(uint8_t *a, int64_t na, uint8_t *b, int64_t nb) {
+  const int64_t step = (int64_t)gridDim.x * blockDim.x, first = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  for (int64_t i = first; i < na; i += step) a[i] = 0;
+  for (int64_t i = first; i < nb; i += step) b[i] = 0;
+}
+
+template <int DT, int TC, bool GATED, bool GATHER, bool ONCE = false>
+void launch_quantize_layout(const QuantParams &p, unsigned blocks, hipStream_t stream) {
+  if (p.scale_layout == WAVE_MXFP4_SCALE_MFMA32)
+    quantize_kernel<DT, TC, GATED, GATHER, WAVE_MXFP4_SCALE_MFMA32, ONCE><<<dim3(blocks), 256, 0, stream>>>(p);
+  else if (p.scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE)
+    quantize_kernel<DT, TC, GATED, GATHER, WAVE_MXFP4_SCALE_E8M0_SHUFFLE, ONCE><<<dim3(blocks), 256, 0, stream>>>(p);
+  else
+    quantize_kernel<DT, TC, GATED, GATHER, WAVE_MXFP4_SCALE_ROW_MAJOR, ONCE><<<dim3(blocks), 256, 0, stream>>>(p);
+}
+
+// Codes from here on are stored with the default policy.  The kernel itself is 2 - 4 % faster with non-temporal stores at any
+// size, but the GEMM that follows reads a large A sooner with the default one: linear calls (quantiser and GEMM) of 6 MB and more
+// take 0.96 - 0.98 of the time on the deep-ring tiles (1153 x 5120 x 11168 68 -> 59 us) and 0.99 - 1.00 on the others; below, 1.01 -
+// 1.02 on the persistent kernel and 1.00 elsewhere.
+constexpr int64_t kQuantStreamBytes = 6 << 20;
+// 16-bit inputs from here on are loaded non-temporal: read once, they would push what the GEMM reads out of the memory-side
+// cache (2048 x 14336 in front of its GEMM with changing operands: 73.4 us, 75.5 with the default policy).  Smaller ones come from
+// the caches, as the kernel before left them: 4096 x 4096 8.9 -> 8.4 us, 1000 x 4096 4.0 -> 3.9; so do a gathered batch, whose rows
+// are read more than once (4096 rows twice 14.4 -> 11.5), the gated form (2048 x 14336 12.5 -> 11.0), and f32, whose two loads
+// share lines.
+constexpr int64_t kQuantOnceBytes = 32 << 20;
+
 template <int DT, bool GATED>
-hipError_t launch_quantize_dt(const QuantParams &p, int num_cus, hipStream_t stream) {
+hipError_t launch_quantize_dt(QuantParams p, hipStream_t stream) {
+  p.stream_q = (int64_t)p.rows * (p.k >> 1) < kQuantStreamBytes;
   const int ks = p.k >> 5;
   const int64_t row_tiles = (p.rows + kQuantRows - 1) / kQuantRows;
   // One K tile (256 columns) per workgroup: many small workgroups keep loads and stores of different rows mixed
@@ -242,12 +283,22 @@ hipError_t launch_quantize_dt(const QuantParams &p, int num_cus, hipStream_t str
   if (narrow > 0x7FFFFFFF) return hipErrorInvalidValue;
   if constexpr (!GATED) {
     if (p.row_ids != nullptr) {
-      quantize_kernel<DT, 2, false><<<dim3((unsigned)pairs), 256, 0, stream>>>(p);
+      if (p.src_rows < 1) {  // no row to load: every id is beyond the last one
+        const int64_t sc = p.scale_layout == WAVE_MXFP4_SCALE_ROW_MAJOR ? (int64_t)p.rows * ks : row_tiles * 32 * ((ks + 7) & ~7);
+        zero_bytes_kernel<<<dim3(256), 256, 0, stream>>>(p.q, (int64_t)p.rows * (p.k >> 1), p.scale, sc);
+        return hipGetLastError();
+      }
+      launch_quantize_layout<DT, 2, false, true>(p, (unsigned)pairs, stream);
       return hipGetLastError();
     }
   }
-  (void)num_cus;
-  quantize_kernel<DT, 1, GATED><<<dim3((unsigned)narrow), 256, 0, stream>>>(p);
+  if constexpr (DT != WAVE_MXFP4_IN_F32 && !GATED) {
+    if ((int64_t)p.rows * p.k * 2 >= kQuantOnceBytes) {
+      launch_quantize_layout<DT, 1, GATED, false, true>(p, (unsigned)narrow, stream);
+      return hipGetLastError();
+    }
+  }
+  launch_quantize_layout<DT, 1, GATED, false>(p, (unsigned)narrow, stream);
   return hipGetLastError();
 }
 
@@ -282,9 +333,9 @@ hipError_t launch_quantize(const void *x, int in_dtype, const int32_t *row_ids, 
   p.ld_x = k, p.rows = (int)rows, p.k = (int)k, p.src_rows = (int)src_rows, p.row_div = row_div > 0 ? row_div : 1;
   p.scale_layout = scale_layout;
   switch (in_dtype) {
-    case WAVE_MXFP4_IN_F32: return launch_quantize_dt<WAVE_MXFP4_IN_F32, false>(p, num_cus, stream);
-    case WAVE_MXFP4_IN_BF16: return launch_quantize_dt<WAVE_MXFP4_IN_BF16, false>(p, num_cus, stream);
-    case WAVE_MXFP4_IN_F16: return launch_quantize_dt<WAVE_MXFP4_IN_F16, false>(p, num_cus, stream);
+    case WAVE_MXFP4_IN_F32: return launch_quantize_dt<WAVE_MXFP4_IN_F32, false>(p, stream);
+    case WAVE_MXFP4_IN_BF16: return launch_quantize_dt<WAVE_MXFP4_IN_BF16, false>(p, stream);
+    case WAVE_MXFP4_IN_F16: return launch_quantize_dt<WAVE_MXFP4_IN_F16, false>(p, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -298,8 +349,8 @@ hipError_t launch_silu_and_mul_quantize(const void *gate, const void *up, int64_
   p.ld_x = ld_gate, p.ld_up = ld_up, p.rows = (int)rows, p.k = (int)n, p.src_rows = (int)rows, p.row_div = 1;
   p.scale_layout = scale_layout;
   switch (in_dtype) {
-    case WAVE_MXFP4_IN_BF16: return launch_quantize_dt<WAVE_MXFP4_IN_BF16, true>(p, num_cus, stream);
-    case WAVE_MXFP4_IN_F16: return launch_quantize_dt<WAVE_MXFP4_IN_F16, true>(p, num_cus, stream);
+    case WAVE_MXFP4_IN_BF16: return launch_quantize_dt<WAVE_MXFP4_IN_BF16, true>(p, stream);
+    case WAVE_MXFP4_IN_F16: return launch_quantize_dt<WAVE_MXFP4_IN_F16, true>(p, stream);
     default: return hipErrorInvalidValue;
   }
 }
