@@ -104,19 +104,22 @@ __global__ void scale_convert_kernel(const uint8_t *__restrict__ src, int src_la
   }
 }
 
-// Row-major -> MFMA32, the conversion in front of every tile GEMM with row-major scales (8-byte reads as two
-// dwords where the rows start on dwords, ks % 4 == 0; byte reads otherwise).  A workgroup takes 32 blocks of (32 rows x one K
-// tile): 32 rows x 32 K tiles, or for short rows 64 x 16 or 128 x 8, so that all
+// Row-major -> MFMA32, the conversion in front of every tile GEMM with row-major scales.  A workgroup takes 32 blocks of (32
+// rows x one K tile): 32 rows x 32 K tiles, or for short rows 64 x 16 or 128 x 8, so that all
 // of its threads have a piece whatever K is (with 16 K tiles a row, K = 4096, half
-// of them had none).  8-byte reads that walk each row contiguously, the even and
+// of them had none).  8-byte reads that walk each row contiguously, wherever the rows start, the even and
 // odd groups of a K tile split with v_perm into the two dwords of its block (lanes
 // r%32 and 32 + r%32), a pass through LDS (block stride 65 dwords), and dword
 // writes that walk the destination contiguously.
+// Bound by latency: one round trip for the four pieces of a thread (us, 8192 x 8192 x 8192's two tensors, kernel trace: 6.8
+// with each piece loaded behind a branch, 6.1; rows that do not start on dwords, formerly a byte at a time: a call of 76 x 1376 x
+// 992 11.0 -> 9.1, 2183 x 1472 x 2208 15.7 -> 13.2, 26 x 22144 x 4928 25.8 -> 22.2).
 // blockIdx.z picks one of two tensors with the same ks (the A and B scales of a
 // GEMM go through one launch; rows of one of them 0 for a single tensor).
 // With gt.table the launch's first workgroup builds the M tile table of a grouped
 // GEMM before its share of the scales (mxfp4_group_table.h): the table only needs
 // the offsets, so it costs the call no launch of its own.
+typedef uint64_t Unaligned64 __attribute__((aligned(1)));
 // K tiles of a row that one workgroup walks, as a power of two: 5, 4 or 3.
 __host__ __device__ inline int scale_wg_kt_log(int k_tiles) { return k_tiles > 16 ? 5 : k_tiles > 8 ? 4 : 3; }
 __global__ void __launch_bounds__(256) scale_to_mfma32_kernel(const uint8_t *__restrict__ src0,
@@ -139,28 +142,44 @@ __global__ void __launch_bounds__(256) scale_to_mfma32_kernel(const uint8_t *__r
   const int row_base = rt0 * 32;
   if (row_base >= rows) return;  // the grid is sized for the taller tensor
   const int t = threadIdx.x;
+  auto stage_block = [&](int unit, uint64_t w) {
+    const int r = unit >> kt_log, blk = ((r >> 5) << kt_log) + (unit & kt_mask);
+    const uint32_t lo = (uint32_t)w, hi = (uint32_t)(w >> 32);
+    stage[blk * 65 + (r & 31)] = __builtin_amdgcn_perm(hi, lo, 0x06040200u);       // groups 0, 2, 4, 6
+    stage[blk * 65 + 32 + (r & 31)] = __builtin_amdgcn_perm(hi, lo, 0x07050301u);  // groups 1, 3, 5, 7
+  };
+  // Every thread loads its four pieces, and all of them are on their way before the first is used: pieces beyond the tensor
+  // from the nearest place inside it, a row's last groups together with what follows them, masked off.
+  const int64_t bytes = (int64_t)rows * ks;
+  if (bytes >= 8) {
+    uint64_t v[4];
+    int shift[4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int unit = t + 256 * u, r = unit >> kt_log, ktl = unit & kt_mask;
-    const int row = row_base + r, kt = kt0 + ktl;
-    uint2 v = make_uint2(0u, 0u);
-    if (row < rows && kt < k_tiles) {
-      const uint8_t *at = src + (int64_t)row * ks + (int64_t)kt * 8;
-      if ((ks & 3) == 0) {
-        v.x = *(const uint32_t *)at;
-        if (kt * 8 + 4 < ks) v.y = *(const uint32_t *)(at + 4);
-      } else {
-        // rows that do not start on dwords (K % 128 != 0): byte by byte, groups past the end of the row stay 0
-        const int valid = min(8, ks - kt * 8);
-        for (int b = 0; b < valid; ++b) {
-          const uint32_t byte = at[b];
-          if (b < 4) v.x |= byte << (8 * b); else v.y |= byte << (8 * (b - 4));
-        }
-      }
+    for (int u = 0; u < 4; ++u) {
+      const int unit = t + 256 * u, r = unit >> kt_log, ktl = unit & kt_mask;
+      const int64_t at = (int64_t)min(row_base + r, rows - 1) * ks + (int64_t)min(kt0 + ktl, k_tiles - 1) * 8;
+      const int64_t from = at < bytes - 8 ? at : bytes - 8;
+      v[u] = *(const Unaligned64 *)(src + from);
+      shift[u] = (int)(at - from) * 8;
     }
-    const int blk = ((r >> 5) << kt_log) + ktl;
-    stage[blk * 65 + (r & 31)] = __builtin_amdgcn_perm(v.y, v.x, 0x06040200u);       // groups 0, 2, 4, 6
-    stage[blk * 65 + 32 + (r & 31)] = __builtin_amdgcn_perm(v.y, v.x, 0x07050301u);  // groups 1, 3, 5, 7
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int unit = t + 256 * u, r = unit >> kt_log, ktl = unit & kt_mask;
+      const int valid = ks - (kt0 + ktl) * 8;  // groups of the row from here on
+      uint64_t w = v[u] >> shift[u];
+      if (valid < 8) w &= valid > 0 ? (1ull << (8 * valid)) - 1 : 0ull;
+      if (row_base + r >= rows) w = 0;
+      stage_block(unit, w);
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int unit = t + 256 * u, row = row_base + (unit >> kt_log);
+      uint64_t w = 0;
+      if (row < rows && (unit & kt_mask) == 0 && kt0 == 0)
+        for (int b = 0; b < ks; ++b) w |= (uint64_t)src[(int64_t)row * ks + b] << (8 * b);
+      stage_block(unit, w);
+    }
   }
   __syncthreads();
   uint32_t *out = (uint32_t *)dst;
@@ -176,6 +195,7 @@ __global__ void __launch_bounds__(256) scale_to_mfma32_kernel(const uint8_t *__r
 // conversion permutes bytes inside a block.  One thread per destination dword (lane (g%2)*32 + r%32, bytes
 // t = 0..3 = groups 2t + g%2): its bytes come from the two source dwords (g%4)*16 + r%16 for g%4 = g%2 and
 // 2 + g%2, byte (g/4)*2 + (r%32)/16 of each.  blockIdx.y picks one of two tensors.
+typedef uint32_t DwordRun __attribute__((ext_vector_type(4), aligned(4)));  // (both tensors start on a dword)
 __global__ void __launch_bounds__(256) scale_shuffle_to_mfma32_kernel(const uint32_t *__restrict__ src0,
                                                                       uint32_t *__restrict__ dst0, int64_t dwords0,
                                                                       const uint32_t *__restrict__ src1,
@@ -183,11 +203,14 @@ __global__ void __launch_bounds__(256) scale_shuffle_to_mfma32_kernel(const uint
   const uint32_t *src = blockIdx.y ? src1 : src0;
   uint32_t *dst = blockIdx.y ? dst1 : dst0;
   const int64_t dwords = blockIdx.y ? dwords1 : dwords0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < dwords; i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t blk = i >> 6;
-    const int lane = (int)(i & 63), r32 = lane & 31, gpar = lane >> 5;
-    const uint32_t d0 = src[blk * 64 + gpar * 16 + (r32 & 15)], d1 = src[blk * 64 + (2 + gpar) * 16 + (r32 & 15)];
-    dst[i] = __builtin_amdgcn_perm(d1, d0, (r32 >> 4) ? 0x07030501u : 0x06020400u);
+  // four dwords per thread: lanes 4 q .. 4 q + 3 of a block, whose sources are two runs of four dwords
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < dwords / 4; i += (int64_t)gridDim.x * blockDim.x) {
+    const int q = (int)(i & 15), gpar = q >> 3;
+    const DwordRun *s = (const DwordRun *)(src + (i >> 4) * 64 + gpar * 16 + (q & 3) * 4);
+    const DwordRun d0 = s[0], d1 = s[8];
+    const uint32_t sel = q & 4 ? 0x07030501u : 0x06020400u;
+    *(DwordRun *)(dst + i * 4) = DwordRun{__builtin_amdgcn_perm(d1.x, d0.x, sel), __builtin_amdgcn_perm(d1.y, d0.y, sel),
+                                          __builtin_amdgcn_perm(d1.z, d0.z, sel), __builtin_amdgcn_perm(d1.w, d0.w, sel)};
   }
 }
 
@@ -376,7 +399,7 @@ hipError_t launch_scale_convert(const uint8_t *src, int src_layout, uint8_t *dst
     return hipGetLastError();
   }
   if (src_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE && dst_layout == WAVE_MXFP4_SCALE_MFMA32 && ((uintptr_t)src & 3) == 0) {
-    scale_shuffle_to_mfma32_kernel<<<dim3(blocks_for(n, kThreads), 1), kThreads, 0, stream>>>(
+    scale_shuffle_to_mfma32_kernel<<<dim3(blocks_for(n / 4, kThreads), 1), kThreads, 0, stream>>>(
         (const uint32_t *)src, (uint32_t *)dst, n, nullptr, nullptr, 0);
     return hipGetLastError();
   }
@@ -391,7 +414,7 @@ hipError_t launch_scale_pair_shuffle_to_mfma32(const uint8_t *a_src, uint8_t *a_
   if ((((uintptr_t)a_src | (uintptr_t)b_src) & 3) != 0) return hipErrorInvalidValue;
   const int64_t ksp = (ks + 7) / 8 * 8;
   const int64_t na = (a_rows + 31) / 32 * 32 * (ksp / 4), nb = (b_rows + 31) / 32 * 32 * (ksp / 4);
-  scale_shuffle_to_mfma32_kernel<<<dim3(blocks_for(na > nb ? na : nb, kThreads), 2), kThreads, 0, stream>>>(
+  scale_shuffle_to_mfma32_kernel<<<dim3(blocks_for((na > nb ? na : nb) / 4, kThreads), 2), kThreads, 0, stream>>>(
       (const uint32_t *)a_src, (uint32_t *)a_dst, na, (const uint32_t *)b_src, (uint32_t *)b_dst, nb);
   return hipGetLastError();
 }
