@@ -436,9 +436,8 @@ hipError_t launch_asym_out(const GemmParams &p, int grid_x, hipStream_t stream) 
 
 }  // namespace
 
-// Whether the asymmetric kernel serves this problem (`forced`: the caller named the variant, so a problem with
-// fewer tiles than CUs is taken too).
-bool asym_gemm_applies(const GemmParams &p, int num_cus, bool forced) {
+// Whether the asymmetric kernel serves this problem, of any number of tiles.
+bool asym_gemm_applies(const GemmParams &p, int num_cus) {
   if (!p.b_preshuffled || p.num_groups != 0 || p.tile_table != nullptr || p.splits != 1 || p.partial != nullptr) return false;
   const bool shuffled = p.a_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE && p.b_scale_layout == WAVE_MXFP4_SCALE_E8M0_SHUFFLE;
   if (!shuffled && (p.a_scale_layout != WAVE_MXFP4_SCALE_MFMA32 || p.b_scale_layout != WAVE_MXFP4_SCALE_MFMA32)) return false;
@@ -446,10 +445,7 @@ bool asym_gemm_applies(const GemmParams &p, int num_cus, bool forced) {
   // 32-bit offsets inside one operand tile and one C tile
   if ((int64_t)256 * p.kp >= ((int64_t)1 << 31) || (int64_t)256 * p.n * 4 >= ((int64_t)1 << 31)) return false;
   if ((int64_t)8 * p.k_tiles * 256 >= ((int64_t)1 << 31)) return false;
-  const int grid = num_cus / kNumXcd * kNumXcd;
-  if (grid < kNumXcd) return false;
-  const int64_t tiles = (int64_t)((p.m + 255) / 256) * (p.n / 256);
-  return forced || tiles > grid;
+  return num_cus >= kNumXcd;
 }
 
 hipError_t launch_asym_gemm(const GemmParams &p, int num_cus, hipStream_t stream) {
