@@ -1,0 +1,46 @@
+"""GPU: calls with row-major scales at the borders where the library's own choice goes to the deep-ring kernel, against the exact
+oracle; and, on the CPU, the kernel on either side of each border."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import c_oracle
+from oracle import mxfp4_oracle as orc
+from wave_amd import _lib
+
+from gpu_util import assert_close, run_gemm
+from test_launch_choice_host import QUERY, launches  # noqa: F401  (a fixture)
+
+ROW, SHUF = _lib.B_ROW_MAJOR, _lib.B_PRESHUFFLE
+# rows, the last shape (N, K tiles) on the deep ring and the first on the other side, B
+BORDERS = [
+    (7, (4096, 13), (4096, 14), ROW), (16, (6144, 32), (6152, 32), ROW), (3, (16384, 20), (16384, 24), ROW),
+    (17, (16384, 5), (16392, 5), ROW), (9, (3080, 35), (8320, 35), ROW), (5, (4096, 9), (4096, 8), SHUF),
+    (12, (6144, 29), (6144, 28), SHUF), (1, (8192, 8), (8192, 10), SHUF), (20, (16384, 20), (16400, 20), SHUF),
+    (32, (12288, 40), (12320, 40), ROW), (90, (8192, 20), (8224, 20), SHUF), (70, (16384, 6), (16416, 6), ROW),
+]
+
+
+def gemm(m, shape, b):
+    return ("gemm", m, shape[0], 256 * shape[1], _lib.OUT_BF16, _lib.SCALE_ROW_MAJOR, _lib.SCALE_ROW_MAJOR, b, 0, 0, QUERY)
+
+
+@pytest.mark.parametrize("m,near,far,b", BORDERS)
+def test_borders(launches, m, near, far, b):  # noqa: F811
+    on, off = launches([gemm(m, near, b), gemm(m, far, b)])
+    assert on.startswith("0 |") and "deep_gemm_kernel" in on and "to_mfma32" not in on, on
+    assert off.startswith("0 |") and "deep_gemm_kernel" not in off, off
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,near,b", [(m, near, b) for m, near, far, b in BORDERS] +
+                         [(130, (12288, 4), SHUF), (256, (13312, 12), SHUF), (2, (1032, 13), ROW), (130, (12264, 5), ROW)])
+def test_staged_rows(m, near, b):
+    n, k = near[0], 256 * near[1]
+    x, xs, w_t, ws = orc.make_inputs(m, n, k, seed=m + n + k, scale_lo=118, scale_hi=136)
+    rows = np.unique(np.r_[0, m // 2, m - 1])
+    ref = c_oracle.scaled_gemm_exact(x, w_t, xs, ws, rows=rows)
+    for out_dtype in (torch.float32, torch.bfloat16):
+        got = run_gemm(x, xs, orc.b_preshuffle(w_t) if b == SHUF else w_t, ws, out_dtype, b_layout=b)
+        assert_close(got[rows], ref, out_dtype, f"{m} x {n} x {k}")
