@@ -1,4 +1,4 @@
-"""GPU: calls with row-major scales at the borders where the library's own choice goes to the deep-ring kernel, against the exact
+"""GPU: calls of few rows at the borders where the library's own choice goes to the deep-ring kernel, against the exact
 oracle; and, on the CPU, the kernel on either side of each border."""
 
 import numpy as np
@@ -10,6 +10,7 @@ from oracle import mxfp4_oracle as orc
 from wave_amd import _lib
 
 from gpu_util import assert_close, run_gemm
+from test_gpu_deep_ring_by_name import CONV, LAYOUT
 from test_launch_choice_host import QUERY, launches  # noqa: F401  (a fixture)
 
 ROW, SHUF = _lib.B_ROW_MAJOR, _lib.B_PRESHUFFLE
@@ -20,15 +21,21 @@ BORDERS = [
     (12, (6144, 29), (6144, 28), SHUF), (1, (8192, 8), (8192, 10), SHUF), (20, (16384, 20), (16400, 20), SHUF),
     (32, (12288, 40), (12320, 40), ROW), (90, (8192, 20), (8224, 20), SHUF), (70, (16384, 6), (16416, 6), ROW),
 ]
+# the same with scales in a blocked order
+BLOCKED = [
+    (16, (6144, 32), (8192, 32), ROW), (2, (8192, 15), (8192, 16), ROW), (7, (12288, 16), (12288, 20), ROW),
+    (1, (9216, 20), (9216, 24), SHUF), (3, (10240, 40), (10240, 48), ROW),
+]
 
 
-def gemm(m, shape, b):
-    return ("gemm", m, shape[0], 256 * shape[1], _lib.OUT_BF16, _lib.SCALE_ROW_MAJOR, _lib.SCALE_ROW_MAJOR, b, 0, 0, QUERY)
+def gemm(m, shape, b, scales):
+    return ("gemm", m, shape[0], 256 * shape[1], _lib.OUT_BF16, scales, scales, b, 0, 0, QUERY)
 
 
-@pytest.mark.parametrize("m,near,far,b", BORDERS)
-def test_borders(launches, m, near, far, b):  # noqa: F811
-    on, off = launches([gemm(m, near, b), gemm(m, far, b)])
+@pytest.mark.parametrize("m,near,far,b,scales", [c + (_lib.SCALE_ROW_MAJOR,) for c in BORDERS] +
+                         [c + (s,) for c in BLOCKED for s in (_lib.SCALE_E8M0_SHUFFLE, _lib.SCALE_MFMA32)])
+def test_borders(launches, m, near, far, b, scales):  # noqa: F811
+    on, off = launches([gemm(m, near, b, scales), gemm(m, far, b, scales)])
     assert on.startswith("0 |") and "deep_gemm_kernel" in on and "to_mfma32" not in on, on
     assert off.startswith("0 |") and "deep_gemm_kernel" not in off, off
 
@@ -43,4 +50,18 @@ def test_staged_rows(m, near, b):
     ref = c_oracle.scaled_gemm_exact(x, w_t, xs, ws, rows=rows)
     for out_dtype in (torch.float32, torch.bfloat16):
         got = run_gemm(x, xs, orc.b_preshuffle(w_t) if b == SHUF else w_t, ws, out_dtype, b_layout=b)
+        assert_close(got[rows], ref, out_dtype, f"{m} x {n} x {k}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,near,b", [(m, near, b) for m, near, far, b in BLOCKED])
+@pytest.mark.parametrize("scales", ["e8m0", "mfma32"])
+def test_blocked_scales(m, near, b, scales):
+    n, k = near[0], 256 * near[1]
+    x, xs, w_t, ws = orc.make_inputs(m, n, k, seed=m + n + k, scale_lo=118, scale_hi=136)
+    rows = np.unique(np.r_[0, m // 2, m - 1])
+    ref = c_oracle.scaled_gemm_exact(x, w_t, xs, ws, rows=rows)
+    for out_dtype in (torch.float32, torch.bfloat16):
+        got = run_gemm(x, CONV[scales](xs), orc.b_preshuffle(w_t) if b == SHUF else w_t, CONV[scales](ws), out_dtype,
+                       a_scale_layout=LAYOUT[scales], b_scale_layout=LAYOUT[scales], b_layout=b)
         assert_close(got[rows], ref, out_dtype, f"{m} x {n} x {k}")
