@@ -158,7 +158,7 @@ class DeepRing:
     """wave_mxfp4_gemm_deep_ring behind the call shape of wave_amd.mxfp4_gemm, for time_gemm: one tile shape and number of
     parts by name, row-major scales staged or re-laid in front."""
 
-    TILES = [(64, 64), (64, 128), (128, 128), (128, 256), (256, 128)]
+    TILES = {0: (64, 64), 1: (64, 128), 2: (128, 128), 3: (128, 256), 4: (256, 128), 8: (128, 192)}  # by its number in the library
 
     def __init__(self, torch, shape, parts, relayout, scratch):
         from wave_amd import _lib
@@ -844,7 +844,7 @@ def main():
                         by_name[f"{name}/{split}"] = round(best_of_two(variant=v, split_k=split), 1)
                     except (RuntimeError, ValueError):
                         pass   # (a split this K does not divide into, or a kernel that does not take the shape)
-            for shape, (bm, bn) in enumerate(DeepRing.TILES):
+            for shape, (bm, bn) in DeepRing.TILES.items():
                 for parts in range(1, 9):
                     for relayout in ((0,) if native else (0, 1)):
                         if not DeepRing.one_round(shape, parts, m, n) or 4 * parts * m * n > scratch.numel() // 2:

@@ -94,7 +94,8 @@ typedef enum {
    * gemm_mxfp4_double_buffer.py:1781-2222).  Needs b_layout PRESHUFFLE,
    * N % 256 == 0, K % 512 == 0, K >= 1536 and either MFMA32 scales or the
    * workspace; WAVE_MXFP4_ERR_UNSUPPORTED otherwise.  AUTO takes it where it
-   * applies and the problem has more tiles than the GPU has CUs. */
+   * applies, the problem has more tiles than half the GPU's CUs and no tile of
+   * the deep-ring kernel covers it in one round. */
   WAVE_MXFP4_VARIANT_T256x256_W1x4_BDIRECT = 7,
   /* M <= 256 against a wide B from HBM: one workgroup per strip of 64 to 128 columns, B through deep
    * wave-private LDS rings, A fed by a producer wave.  Needs K > 768, N % 4 == 0, no split, and
