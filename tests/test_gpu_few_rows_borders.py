@@ -42,7 +42,7 @@ def test_borders(launches, m, near, far, b, scales):  # noqa: F811
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,near,b", [(m, near, b) for m, near, far, b in BORDERS] +
-                         [(130, (12288, 4), SHUF), (256, (13312, 12), SHUF), (2, (1032, 13), ROW), (130, (12264, 5), ROW)])
+                         [(2, (1032, 13), ROW), (130, (12264, 5), ROW)])
 def test_staged_rows(m, near, b):
     n, k = near[0], 256 * near[1]
     x, xs, w_t, ws = orc.make_inputs(m, n, k, seed=m + n + k, scale_lo=118, scale_hi=136)
