@@ -26,25 +26,32 @@ BLOCKED = [
     (16, (6144, 32), (8192, 32), ROW), (2, (8192, 15), (8192, 16), ROW), (7, (12288, 16), (12288, 20), ROW),
     (1, (9216, 20), (9216, 24), SHUF), (3, (10240, 40), (10240, 48), ROW),
 ]
+# row-major scales and a partial last K tile, which a launch in front re-lays for the deep ring (K tiles in parts of one)
+TAILS = [
+    (3, (4096, 5.5), (4096, 6.5), ROW), (40, (2048, 10.125), (2048, 11.125), ROW), (16, (8192, 15.125), (8192, 16.125), ROW),
+    (1, (11968, 22.875), (11968, 23.125), ROW), (17, (4104, 31.5), (4096, 31.5), ROW), (8, (6144, 39.5), (6144, 38.5), ROW),
+    (100, (16384, 7.5), (16392, 7.5), ROW),
+]
 
 
 def gemm(m, shape, b, scales):
-    return ("gemm", m, shape[0], 256 * shape[1], _lib.OUT_BF16, scales, scales, b, 0, 0, QUERY)
+    return ("gemm", m, shape[0], int(256 * shape[1]), _lib.OUT_BF16, scales, scales, b, 0, 0, QUERY)
 
 
 @pytest.mark.parametrize("m,near,far,b,scales", [c + (_lib.SCALE_ROW_MAJOR,) for c in BORDERS] +
-                         [c + (s,) for c in BLOCKED for s in (_lib.SCALE_E8M0_SHUFFLE, _lib.SCALE_MFMA32)])
+                         [c + (s,) for c in BLOCKED for s in (_lib.SCALE_E8M0_SHUFFLE, _lib.SCALE_MFMA32)] +
+                         [c + (_lib.SCALE_ROW_MAJOR,) for c in TAILS])
 def test_borders(launches, m, near, far, b, scales):  # noqa: F811
     on, off = launches([gemm(m, near, b, scales), gemm(m, far, b, scales)])
-    assert on.startswith("0 |") and "deep_gemm_kernel" in on and "to_mfma32" not in on, on
+    assert on.startswith("0 |") and "deep_gemm_kernel" in on and ("to_mfma32" in on) == (near[1] % 1 != 0), on
     assert off.startswith("0 |") and "deep_gemm_kernel" not in off, off
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,near,b", [(m, near, b) for m, near, far, b in BORDERS] +
+@pytest.mark.parametrize("m,near,b", [(m, near, b) for m, near, far, b in BORDERS + TAILS] +
                          [(2, (1032, 13), ROW), (130, (12264, 5), ROW)])
-def test_staged_rows(m, near, b):
-    n, k = near[0], 256 * near[1]
+def test_row_major_scales(m, near, b):
+    n, k = near[0], int(256 * near[1])
     x, xs, w_t, ws = orc.make_inputs(m, n, k, seed=m + n + k, scale_lo=118, scale_hi=136)
     rows = np.unique(np.r_[0, m // 2, m - 1])
     ref = c_oracle.scaled_gemm_exact(x, w_t, xs, ws, rows=rows)
@@ -57,7 +64,7 @@ def test_staged_rows(m, near, b):
 @pytest.mark.parametrize("m,near,b", [(m, near, b) for m, near, far, b in BLOCKED])
 @pytest.mark.parametrize("scales", ["e8m0", "mfma32"])
 def test_blocked_scales(m, near, b, scales):
-    n, k = near[0], 256 * near[1]
+    n, k = near[0], int(256 * near[1])
     x, xs, w_t, ws = orc.make_inputs(m, n, k, seed=m + n + k, scale_lo=118, scale_hi=136)
     rows = np.unique(np.r_[0, m // 2, m - 1])
     ref = c_oracle.scaled_gemm_exact(x, w_t, xs, ws, rows=rows)
