@@ -221,3 +221,13 @@ def test_b_direct_variant_rejects_what_it_does_not_take():
     assert gemm(lib, **dict(ok, k=1024)) == _lib.ERR_UNSUPPORTED
     assert gemm(lib, **dict(ok, split=2)) in (_lib.ERR_UNSUPPORTED, _lib.ERR_WORKSPACE)
     assert gemm(lib, **dict(ok, asl=0)) == _lib.ERR_UNSUPPORTED       # row-major scales need the workspace
+
+
+@pytest.mark.parametrize("shape", [-1, 1, 3, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("a_fmt,b_fmt", [(0, 0), (1, 0), (0, 2), (2, 1)])
+@pytest.mark.parametrize("relayout", [0, 1])
+def test_deep_ring_refuses_tiles_that_mxfp8_is_not_built_for(shape, a_fmt, b_fmt, relayout):
+    """... before anything is launched into the caller's scratch."""
+    lib = _lib.load()
+    assert lib.wave_mxfp4_gemm_deep_ring(P, P, P, P, P, 64, 64, 1024, a_fmt, b_fmt, 0, _lib.SCALE_ROW_MAJOR, 0, shape, 1, relayout,
+                                         P if relayout else None, 1 << 20, None) == _lib.ERR_UNSUPPORTED

@@ -76,6 +76,16 @@ R with_deep_shape(int shape, R none, F f) {
     default: return none;
   }
 }
+// ... and those that are built for MXFP8 operands (kDeepShapes8)
+template <class R, class F>
+R with_deep8_shape(int shape, R none, F f) {
+  switch (shape) {
+    case 0: return f(DeepCfg<64, 64, 2, 2, 4>{});
+    case 2: return f(DeepCfg<128, 128, 2, 4, 4>{});
+    case 4: return f(DeepCfg<256, 128, 4, 2, 3>{});
+    default: return none;
+  }
+}
 // K tiles of row-major scales a workgroup can stage behind the ring: `unit` bytes per row and K tile (8, MXFP8: 4), rows
 // padded to an odd count of units (conflict-free reads).
 template <class Cfg>

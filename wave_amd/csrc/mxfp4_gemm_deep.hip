@@ -35,7 +35,8 @@ hipError_t launch_deep_gemm(const GemmParams &p, int shape, hipStream_t stream) 
 }
 
 int deep_rows_max(int shape, bool fp8) {
-  return with_deep_shape(shape, 0, [&](auto cfg) { return fp8 ? rows_max_k_tiles<decltype(cfg)>(4) : rows_max_k_tiles<DeepRowsCfg<decltype(cfg)>>(8); });
+  if (fp8) return with_deep8_shape(shape, 0, [](auto cfg) { return rows_max_k_tiles<decltype(cfg)>(4); });
+  return with_deep_shape(shape, 0, [](auto cfg) { return rows_max_k_tiles<DeepRowsCfg<decltype(cfg)>>(8); });
 }
 
 }  // namespace wave_mxfp4

@@ -37,12 +37,8 @@ hipError_t launch_deep8_formats(const GemmParams &p, int a_fmt, int b_fmt, hipSt
 }  // namespace
 
 hipError_t launch_deep_gemm_fp8(const GemmParams &p, int shape, int a_fmt, int b_fmt, hipStream_t stream) {
-  switch (shape) {
-    case 0: return launch_deep8_formats<DeepCfg<64, 64, 2, 2, 4>>(p, a_fmt, b_fmt, stream);
-    case 2: return launch_deep8_formats<DeepCfg<128, 128, 2, 4, 4>>(p, a_fmt, b_fmt, stream);
-    case 4: return launch_deep8_formats<DeepCfg<256, 128, 4, 2, 3>>(p, a_fmt, b_fmt, stream);
-    default: return hipErrorInvalidValue;
-  }
+  return with_deep8_shape(shape, hipErrorInvalidValue,
+                          [&](auto cfg) { return launch_deep8_formats<decltype(cfg)>(p, a_fmt, b_fmt, stream); });
 }
 
 }  // namespace wave_mxfp4
