@@ -162,11 +162,10 @@ int persist_tail_parts(const GemmParams &p, int variant, int num_cus, size_t *pa
 hipError_t launch_skinny_gemm(const GemmParams &p, hipStream_t stream);
 hipError_t launch_scale_spread_rows(const uint8_t *src, uint8_t *dst, int64_t rows, int64_t ks, hipStream_t stream);
 hipError_t launch_quantize(const void *x, int in_dtype, const int32_t *row_ids, int row_div, int64_t src_rows,
-                           uint8_t *q, uint8_t *scale, int64_t rows, int64_t k, int scale_layout, int num_cus,
-                           hipStream_t stream);
+                           uint8_t *q, uint8_t *scale, int64_t rows, int64_t k, int scale_layout, hipStream_t stream);
 hipError_t launch_silu_and_mul_quantize(const void *gate, const void *up, int64_t ld_gate, int64_t ld_up, int in_dtype,
                                         uint8_t *q, uint8_t *scale, int64_t rows, int64_t n, int scale_layout,
-                                        int num_cus, hipStream_t stream);
+                                        hipStream_t stream);
 hipError_t launch_silu_and_mul(const void *gate, const void *up, void *out, int64_t ld_gate, int64_t ld_up,
                                int64_t ld_out, int in_dtype, int64_t rows, int64_t n, hipStream_t stream);
 constexpr int kMoeMaxExperts = 1024;  // experts the alignment kernel keeps counters for in LDS

@@ -325,8 +325,7 @@ __global__ void __launch_bounds__(256) silu_and_mul_kernel(const uint8_t *__rest
 }  // namespace
 
 hipError_t launch_quantize(const void *x, int in_dtype, const int32_t *row_ids, int row_div, int64_t src_rows,
-                           uint8_t *q, uint8_t *scale, int64_t rows, int64_t k, int scale_layout, int num_cus,
-                           hipStream_t stream) {
+                           uint8_t *q, uint8_t *scale, int64_t rows, int64_t k, int scale_layout, hipStream_t stream) {
   if (rows > 0x7FFFFFFF || k > 0x7FFFFFFF || src_rows > 0x7FFFFFFF) return hipErrorInvalidValue;
   QuantParams p = {};
   p.x = (const uint8_t *)x, p.row_ids = row_ids, p.q = q, p.scale = scale;
@@ -342,7 +341,7 @@ hipError_t launch_quantize(const void *x, int in_dtype, const int32_t *row_ids, 
 
 hipError_t launch_silu_and_mul_quantize(const void *gate, const void *up, int64_t ld_gate, int64_t ld_up, int in_dtype,
                                         uint8_t *q, uint8_t *scale, int64_t rows, int64_t n, int scale_layout,
-                                        int num_cus, hipStream_t stream) {
+                                        hipStream_t stream) {
   if (rows > 0x7FFFFFFF || n > 0x7FFFFFFF) return hipErrorInvalidValue;
   QuantParams p = {};
   p.x = (const uint8_t *)gate, p.up = (const uint8_t *)up, p.q = q, p.scale = scale;
