@@ -95,6 +95,16 @@ def test_scale_convert_every_layout_pair(rows, ks):
     assert np.array_equal(got.view(np.uint32), orc.dequant_f32(q, s2).view(np.uint32))
 
 
+@pytest.mark.parametrize("offset", [0, 1, 3])
+@pytest.mark.parametrize("rows,ks", [(1, 1), (1, 7), (2, 3), (1, 8), (33, 9), (65, 63), (129, 65), (40, 130), (70, 257), (130, 64)])
+def test_row_major_scales_that_start_anywhere(rows, ks, offset):
+    """Row-major -> MFMA32: rows that do not start on dwords, tensors of less than one 8-byte read, a storage offset of bytes."""
+    s = np.random.default_rng(rows * 11 + ks).integers(0, 256, size=(rows, ks), dtype=np.uint8)
+    (flat,) = to_gpu(np.r_[np.full(offset, 0xA5, np.uint8), s.reshape(-1)])
+    got = wave_amd.scale_convert(flat[offset:].view(rows, ks), rows, ks, _lib.SCALE_ROW_MAJOR, _lib.SCALE_MFMA32)
+    assert np.array_equal(got.cpu().numpy(), orc.mfma32_scale_layout(s))
+
+
 @pytest.mark.parametrize("n,kp", [(16, 32), (6144, 3584), (48, 96)])
 def test_b_preshuffle_matches_oracle(n, kp):
     rng = np.random.default_rng(n + kp)

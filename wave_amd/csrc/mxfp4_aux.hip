@@ -390,8 +390,8 @@ hipError_t launch_scale_convert(const uint8_t *src, int src_layout, uint8_t *dst
   const int64_t rows_p = (rows + 31) / 32 * 32, ksp = (ks + 7) / 8 * 8;
   const int64_t n = rows_p * (ksp / 4);
   if (n == 0) return hipSuccess;
-  if (src_layout == WAVE_MXFP4_SCALE_ROW_MAJOR && dst_layout == WAVE_MXFP4_SCALE_MFMA32 && (ks & 3) == 0 &&
-      ((uintptr_t)src & 3) == 0 && rows < ((int64_t)1 << 31) && (ksp / 8 + 31) / 32 <= 65535) {
+  if (src_layout == WAVE_MXFP4_SCALE_ROW_MAJOR && dst_layout == WAVE_MXFP4_SCALE_MFMA32 && rows < ((int64_t)1 << 31) &&
+      (ksp / 8 + 31) / 32 <= 65535) {
     const int kt_log = scale_wg_kt_log((int)(ksp / 8));
     const int64_t rows_wg = 1024 >> kt_log, per_wg = (int64_t)1 << kt_log;  // rows and K tiles a workgroup takes
     dim3 grid((unsigned)((rows + rows_wg - 1) / rows_wg), (unsigned)((ksp / 8 + per_wg - 1) / per_wg), 1);
@@ -431,10 +431,7 @@ hipError_t launch_scale_pair_to_mfma32(const uint8_t *a_src, uint8_t *a_dst, int
     b_rows = 0;
   }
   const int64_t rows_max = a_rows > b_rows ? a_rows : b_rows;
-  // (dword reads where the rows start on dwords, byte reads otherwise)
-  const bool dwords = (ks & 3) == 0;
-  if (ks == 0 || (dwords && (((uintptr_t)a_src & 3) != 0 || (b_rows > 0 && ((uintptr_t)b_src & 3) != 0))) ||
-      rows_max >= ((int64_t)1 << 31) || ((ks + 7) / 8 + 31) / 32 > 65535 || a_rows <= 0 || b_rows < 0)
+  if (ks == 0 || rows_max >= ((int64_t)1 << 31) || ((ks + 7) / 8 + 31) / 32 > 65535 || a_rows <= 0 || b_rows < 0)
     return hipErrorInvalidValue;
   const int kt_log = scale_wg_kt_log((int)((ks + 7) / 8));
   const int64_t rows_wg = 1024 >> kt_log;  // rows a workgroup takes
