@@ -231,3 +231,11 @@ def test_deep_ring_refuses_tiles_that_mxfp8_is_not_built_for(shape, a_fmt, b_fmt
     lib = _lib.load()
     assert lib.wave_mxfp4_gemm_deep_ring(P, P, P, P, P, 64, 64, 1024, a_fmt, b_fmt, 0, _lib.SCALE_ROW_MAJOR, 0, shape, 1, relayout,
                                          P if relayout else None, 1 << 20, None) == _lib.ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("shape,most", [(0, 15), (1, 15), (2, 15), (3, 5), (4, 5), (8, 15)])
+def test_deep_ring_by_name_refuses_more_staged_rows_than_it_names(shape, most):
+    lib = _lib.load()
+    for kt, parts in ((most + 1, 1), (2 * most + 1, 2)):
+        assert lib.wave_mxfp4_gemm_deep_ring(P, P, P, P, P, 64, 64, 256 * kt, 2, 2, 0, _lib.SCALE_ROW_MAJOR, 0, shape, parts, 0, P,
+                                             1 << 20, None) == _lib.ERR_UNSUPPORTED

@@ -56,6 +56,17 @@ def test_128x192(m, n, scales, kt, parts, short, preshuffled, out_dtype):
     assert_close(got, ref, out_dtype, f"{m} x {n} x {k}")
 
 
+@pytest.mark.parametrize("kt", [12, 14, 15])
+@pytest.mark.parametrize("preshuffled", [0, 1])
+def test_128x192_stages_up_to_15_k_tiles(kt, preshuffled):
+    m, n, k = 135, 240, 256 * kt
+    x, xs, w_t, ws = orc.make_inputs(m, n, k, seed=kt, scale_lo=110, scale_hi=140)
+    ref = c_oracle.scaled_gemm_exact(x, w_t, xs, ws)
+    for out_dtype in (torch.float32, torch.bfloat16):
+        got = deep_ring(x, xs, orc.b_preshuffle(w_t) if preshuffled else w_t, ws, out_dtype, k, E2M1, E2M1, "rows", preshuffled, 8, 1)
+        assert_close(got, ref, out_dtype, f"{m} x {n} x {k}")
+
+
 @pytest.mark.parametrize("m,n", [(40, 1024), (130, 2056), (250, 5000), (520, 5624)])
 @pytest.mark.parametrize("kt", [16, 17, 30, 31])
 def test_staged_rows_of_a_long_k(m, n, kt):
