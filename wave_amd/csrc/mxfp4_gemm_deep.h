@@ -12,7 +12,7 @@
 //     ones on these tiles take 0.94 of the time);
 //   * the scales travel in the ring too (one 256-byte block per 32 rows and K tile, four bytes per lane), so that no
 //     load that returns to a register stands in the queue in front of the operands; row-major scales of up to 31 K tiles
-//     (the largest tiles: 5, 128x192: 11) are staged once per workgroup instead, and then no launch has to re-lay them
+//     (the largest tiles: 5, 128x192: 15) are staged once per workgroup instead, and then no launch has to re-lay them
 //     (186 x 4832 x 5888 17.0 -> 10.9 us, 644 x 5888 x 2304 17.1 -> 12.0);
 //   * the tiles are small enough for the problem to reach most CUs without a split along K (64x64 up to 256 of them),
 //     which saves the launch that adds the parts, and the parts.
@@ -93,6 +93,8 @@ __host__ __device__ constexpr int rows_max_k_tiles(int unit) {
   const int units = (160 * 1024 - Cfg::RING) / ((Cfg::BM + Cfg::BN) * unit), odd = units - 1 + units % 2;
   return odd < 31 ? odd : 31;
 }
+static_assert(rows_max_k_tiles<DeepCfg<128, 192, 4, 2, 3>>(8) == 15 && rows_max_k_tiles<DeepCfg<128, 256, 2, 4, 3>>(8) == 5 &&
+              rows_max_k_tiles<DeepCfg<256, 128, 4, 2, 3>>(8) == 5, "as the head of this file has it");
 
 __host__ __device__ constexpr int rows_pitch(int nkt, int unit) { return (nkt + 1 - (nkt & 1)) * unit; }
 
