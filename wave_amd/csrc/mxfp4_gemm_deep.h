@@ -29,10 +29,12 @@
 // sums meet in LDS) were no faster than the even ones beside them, and are not built.
 // Eight waves (two per SIMD) beat four on 128x128 by 1-4 % and on 128x256 by 3-9 %; 64x256 tiles and more than one round
 // (two workgroups of the tile kernel share a CU there, and the persistent kernel streams across tiles) lost and are not
-// built.  A time per K tile of 0.22-0.31 us at 64x64 up to 1.05 at 128x256 leaves the fixed part (launch, first K tile,
-// C: 3.5-5.7 us) as what bounds short K.  On a full grid of the largest tiles it is the step: 2048 x 4096 x 14336 takes 65 us on
-// random operands and 51 on zeros (256x128: 63 and 51), so a fifth is the matrix pipes' power limit; the rest is the lines a CU
-// fetches: its vector L1 keeps about 90 of 128 bytes under way, 512 cycles each (0.18 a cycle), however deep the ring.
+// built.  A time per K tile of 0.21-0.30 us at 64x64 up to 0.93 at 128x256 leaves the fixed part (launch, first K tile,
+// C: 3.3-6.7 us) as what bounds short K.  On a full grid of the largest tiles it is the step: 2048 x 4096 x 14336 takes 65 us on
+// random operands and 54 on zeros (256x128: 66 and 56; 61 and 51 on a faster card), 1000 x 7168 x 4096 22.5 and 17.2, so a fifth to a quarter
+// is the matrix pipes' power limit.  What holds the rest is not established.  It is no limit of a CU's L1 or of what stands
+// behind it: 67 lines of 128 bytes are under way and 0.185 arrive a cycle, where the same requests alone reach 144 and 0.42; no
+// bank conflicts, MFMAs busy 46 % of the cycles (profiles/pmc_deep_ring_l1_requests.txt).
 #ifndef WAVE_MXFP4_GEMM_DEEP_H_
 #define WAVE_MXFP4_GEMM_DEEP_H_
 #include <type_traits>
