@@ -1,6 +1,6 @@
 """GPU: row-major scales that the deep-ring kernel's workgroups stage themselves, at the edges of that staging: every count
 of K tiles from one up (the K tile and the row of a staged piece come from a multiplication in place of a division), up to
-the most that a tile shape takes; the deeper ring that few rows against a long K run on, on both sides of its border; and the
+the most that the call by name takes; the deeper ring that few rows against a long K run on, on both sides of its border; and the
 128x192 tile.
 Against the exact oracle on a sample of rows, with the contract's bounds."""
 
@@ -16,7 +16,7 @@ from test_gpu_deep_ring_by_name import CONV, E2M1, TILES, deep_ring
 
 pytestmark = pytest.mark.gpu
 
-MOST = [15, 15, 15, 5, 5]  # K tiles that every build of the shape has room for
+MOST = [15, 15, 15, 5, 5]  # (the library's own choice stages up to 31: test_gpu_staged_rows_by_choice.py)
 
 
 @pytest.mark.parametrize("shape,kt", [(s, kt) for s in range(5) for kt in sorted({1, 2, 3, 6, 7, 9, 13, 14, 15}) if kt <= MOST[s]])
